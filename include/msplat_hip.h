@@ -101,7 +101,7 @@ int msplat_hip_memset(msplat_hip_ctx *ctx, void *dst, int value, size_t bytes);
 
 /* ── render and train (bindings.h:81-118) ───────────────────────────────────── */
 
-/* msplat_render (bindings.h:81-91): projection + SH, (tile|depth) sort, forward
+/* msplat_render (bindings.h:81-91): projection + SH, depth sort, tile lists, forward
  * compositing. background: host float[3]. *out_img receives the context's cached
  * (H, W, 3) image (device), valid until the next call. */
 int msplat_hip_render(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, const msplat_hip_camera *cam,
@@ -187,9 +187,8 @@ int msplat_hip_render_backward(msplat_hip_ctx *ctx, const msplat_hip_gaussians *
  * Device pointers to the intermediate buffers of the last render/train call, for tests
  * and tools. Per gaussian: xys (N,2) as float4 records (x, y, conic.x, conic.y) and
  * (conic.z, sigmoid(opacity), r, g) plus blue (N), depths, radii, aabb (N,2), tile
- * counts, prefix offsets. Per intersection (sorted): keys (tile<<32 | depth bits,
- * filled by frame_view when MSPLAT_FRAME_KEYS64 is set, else NULL), gaussian ids (NULL
- * without MSPLAT_FRAME_KEYS64 when MSPLAT_TUNE_PACK_KEYS packed them into the sort keys).
+ * counts, prefix offsets (in id order). Per intersection (sorted): keys (tile<<32 | depth
+ * bits, filled by frame_view when MSPLAT_FRAME_KEYS64 is set, else NULL), gaussian ids.
  * tile_start (T+1): tile t owns sorted intersections [tile_start[t], tile_start[t+1]).
  * Per pixel: image, final_T, final_idx (index into
  * the sorted intersections), dL/d(image). Per gaussian reduced gradients (N,2)/(N,3)/
@@ -221,8 +220,7 @@ typedef struct {
     uint64_t *visible_running;
 } msplat_hip_frame;
 int msplat_hip_frame_view(msplat_hip_ctx *ctx, msplat_hip_frame *out);
-/* KEEP_GRADS: fill the reduced gradients; KEYS64: materialise isect_keys on frame_view
- * (and isect_gid, when the tile sort packed the ids into its keys). */
+/* KEEP_GRADS: fill the reduced gradients; KEYS64: materialise isect_keys on frame_view. */
 enum { MSPLAT_FRAME_KEEP_GRADS = 1, MSPLAT_FRAME_KEYS64 = 2 };
 int msplat_hip_set_flags(msplat_hip_ctx *ctx, int flags);
 
@@ -237,10 +235,8 @@ int msplat_hip_set_flags(msplat_hip_ctx *ctx, int flags);
  *                          alpha >= 1/255 ellipse (widened for float rounding) misses
  *                          the tile; 0: every listed gaussian is visited. Skipped pairs
  *                          would composite nothing, so both give identical results.
- *   MSPLAT_TUNE_PACK_KEYS  1 (default): when the tile-id and gaussian-id bits fit in 32,
- *                          the one-view tile sort moves (tile << id bits | id) keys alone
- *                          instead of tile keys plus id values (same order, half the
- *                          bytes); 0: always keys plus values.
+ *   MSPLAT_TUNE_PACK_KEYS  0 or 1 (default 1); without effect, kept for callers that set
+ *                          it: the tiles' lists are built without sort keys.
  *   MSPLAT_TUNE_CHUNKS     depth chunks per tile of the one-view rasterizers (the depth-
  *                          chunked form of msplat_metal.mm:782-907 for views with few
  *                          tiles): 0 (default) picks per frame (fewer than 400 tiles:

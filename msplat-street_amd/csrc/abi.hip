@@ -89,35 +89,35 @@ int do_project(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, const msplat_
 }
 
 // Count scans and their read-back (M intersections, V visible gaussians), then the
-// visible gaussians sorted by depth, keys emitted in that order, the stable tile sort
-// and the tile ranges. The host waits for the counts only after the depth sort and
-// the offsets are enqueued (those run on device-side counts against the gaussian
-// capacity), so the device sorts while the host reads M and sizes the key buffers.
+// visible gaussians sorted by depth and expanded into the tiles' lists. The host waits for
+// the counts only after everything that does not need the intersection buffers is
+// enqueued (the depth sort and the supertile counts run on device-side counts against the
+// gaussian capacity), so the device sorts while the host reads M and sizes the buffers.
 // With an intersection capacity `cap` (a captured step) nothing is read back: every
 // launch after the counts is sized for the capacity and reads the device-side count,
-// and a frame over capacity sets the overflow word and leaves an empty tile list.
+// and a frame over capacity sets the overflow word and leaves empty tile lists.
 int do_bin(msplat_hip_ctx *ctx, uint32_t cap = 0) {
     if (ctx->frame_stage < msplat_hip_ctx::FRAME_PROJECTED)
         return set_error(MSPLAT_ERR_ARG, "binning needs a projected frame on this context");
-    ctx->frame_stage = msplat_hip_ctx::FRAME_PROJECTED;  // the key buffers are rewritten below
+    ctx->frame_stage = msplat_hip_ctx::FRAME_PROJECTED;  // the lists are rewritten below
     const int n = ctx->n;
     const uint32_t nblocks = (uint32_t)((n + 255) / 256);
     if (!ctx->h_total) HIPCHECK(hipHostMalloc((void **)&ctx->h_total, 128, hipHostMallocDefault));
     if (!ctx->counts_ready) HIPCHECK(hipEventCreateWithFlags(&ctx->counts_ready, hipEventDisableTiming));
     const size_t Nc = n > 0 ? (size_t)n : 1;
-    const uint32_t vblocks = (uint32_t)((Nc + 255) / 256);  // depth-ordered list blocks, at most
-    CHECKED(ctx->grow(ctx->scan_part, 4 * 3 * scan_partial_words(std::max(nblocks, vblocks)) + 64));
-    CHECKED(ctx->grow(ctx->hist, 4 * radix_hist_words((uint32_t)std::max<size_t>(Nc, ctx->M > 0 ? ctx->M : 1))));
+    const uint32_t ntiles = (uint32_t)ctx->ntiles, nodes = tile_list_nodes(ctx->tiles_x, ctx->tiles_y);
+    const size_t pw = scan_partial_words(std::max(nblocks, ntiles + 1));
+    CHECKED(ctx->grow(ctx->scan_part, 4 * 2 * pw + 64));
+    CHECKED(ctx->grow(ctx->hist, 4 * radix_hist_words((uint32_t)Nc)));
     CHECKED(ctx->grow(ctx->digit_total, 4 * 256));
     CHECKED(ctx->grow(ctx->dk0, 4 * Nc));
     CHECKED(ctx->grow(ctx->dk1, 4 * Nc));
     CHECKED(ctx->grow(ctx->dv0, 4 * Nc));
     CHECKED(ctx->grow(ctx->dv1, 4 * Nc));
-    CHECKED(ctx->grow(ctx->ord_sums, 4 * (size_t)(vblocks + 1)));
-    CHECKED(ctx->grow(ctx->loff, 4 * Nc));
-    CHECKED(ctx->grow(ctx->tile_start, 4 * (size_t)(ctx->ntiles + 1)));
+    CHECKED(ctx->grow(ctx->lrect, 8 * Nc));
+    CHECKED(ctx->grow(ctx->lists, 4 * tile_list_scratch_words(nodes)));
+    CHECKED(ctx->grow(ctx->tile_start, 4 * (size_t)(ntiles + 1)));
     uint32_t *part = (uint32_t *)ctx->scan_part.p;
-    const size_t pw = scan_partial_words(std::max(nblocks, vblocks));
     hipStream_t s = ctx->stream;
     const ScanOut isects = cap ? ScanOut{ctx->d_total64(), ctx->d_total32(), cap, ctx->d_overflow(), ctx->d_big_count(),
                                          ctx->d_applied(), ctx->d_isects_running()}
@@ -141,9 +141,12 @@ int do_bin(msplat_hip_ctx *ctx, uint32_t cap = 0) {
     c.count = (const uint32_t *)ctx->count.p;
     c.depths = (const float *)ctx->depths.p;
     c.block_vis = (const uint32_t *)ctx->block_vis.p;
+    c.block_sums = (const uint32_t *)ctx->block_sums.p;
     c.dkeys = (uint32_t *)ctx->dk0.p;
     c.dvals = (int32_t *)ctx->dv0.p;
+    c.offsets = (uint32_t *)ctx->offsets.p;
     launch_compact(c, s);
+    ctx->big_listed = false;
     uint32_t *dki = (uint32_t *)ctx->dk0.p, *dko = (uint32_t *)ctx->dk1.p;
     int32_t *dvi = (int32_t *)ctx->dv0.p, *dvo = (int32_t *)ctx->dv1.p;
     for (int shift = 0; shift < 32; shift += 8) {
@@ -153,85 +156,42 @@ int do_bin(msplat_hip_ctx *ctx, uint32_t cap = 0) {
         std::swap(dvi, dvo);
     }
     ctx->vis_sorted = dvi;
-    // intersection offsets in depth order
-    launch_order_sums(dvi, ctx->d_vis32(), (uint32_t)Nc, (const uint32_t *)ctx->count.p, (uint32_t *)ctx->ord_sums.p,
-                      (uint32_t *)ctx->loff.p, s);
-    KeygenArgs k;
-    memset(&k, 0, sizeof k);
-    k.list = dvi;
-    k.nvis_ptr = ctx->d_vis32();
-    k.nvis_max = (uint32_t)Nc;
-    k.count = (const uint32_t *)ctx->count.p;
-    k.rect = (const uint2 *)ctx->rect.p;
-    // up to 4096 chunks the key generation adds the preceding chunk sums itself (a few
-    // loads per thread); past that, one scan launch is cheaper than the quadratic reads
-    if (vblocks <= 4096) {
-        k.chunk_sums = (const uint32_t *)ctx->ord_sums.p;
-    } else {
-        launch_scan_u32((uint32_t *)ctx->ord_sums.p, vblocks, part + 2 * pw,
-                        ScanOut{nullptr, nullptr, 0xFFFFFFFFu, nullptr, nullptr}, s);
-        k.block_bases = (const uint32_t *)ctx->ord_sums.p;
-    }
-    k.offsets = (uint32_t *)ctx->offsets.p;
-    k.loff = (uint32_t *)ctx->loff.p;
-    k.m_ptr = ctx->d_total32();
-    k.big_list = ctx->big_list();
-    k.big_count = ctx->d_big_count();
-    k.tiles_x = ctx->tiles_x;
-    k.overflow = cap ? ctx->d_overflow() : nullptr;
-    launch_keygen_offsets(k, s);
+    // the tiles' lists
+    TileListArgs t;
+    memset(&t, 0, sizeof t);
+    t.list = dvi;
+    t.nvis = ctx->d_vis32();
+    t.overflow = cap ? ctx->d_overflow() : nullptr;
+    t.rect = (const uint2 *)ctx->rect.p;
+    t.lrect = (uint2 *)ctx->lrect.p;
+    t.tile_start = (int32_t *)ctx->tile_start.p;
+    t.direct = tile_list_direct(ctx->tiles_x, ctx->tiles_y);
+    t.tiles_x = ctx->tiles_x;
+    t.tiles_y = ctx->tiles_y;
+    t.nodes = (int)nodes;
+    tile_list_carve((uint32_t *)ctx->lists.p, nodes, t);
+    launch_tile_lists_begin(t, false, nodes, (uint32_t)n, s);
     HIPCHECK(hipGetLastError());
-    // the counts (or the capacity): size the key buffers, then keys (tile ids), stable
-    // tile sort, ranges
-    uint64_t M = cap;
+    // the counts (or the capacity): size the intersection buffers
+    uint64_t M = cap, V = (uint64_t)n;
     if (!cap) {
         HIPCHECK(hipEventSynchronize(ctx->counts_ready));
         ctx->collect();
         M = ctx->h_total[0];
+        V = ctx->h_total[5];
         if (M > 0x7FFFFFFFull)
             return set_error(MSPLAT_ERR_RANGE, "more than 2^31 tile intersections (%llu); lower the resolution",
                              (unsigned long long)M);
         ctx->M = (int64_t)M;
-        ctx->V = (int64_t)ctx->h_total[5];
+        ctx->V = (int64_t)V;
     }
     const size_t Mc = M > 0 ? M : 1;
-    CHECKED(ctx->grow(ctx->keys0, 4 * Mc));
-    CHECKED(ctx->grow(ctx->keys1, 4 * Mc));
-    CHECKED(ctx->grow(ctx->vals0, 4 * Mc));
-    CHECKED(ctx->grow(ctx->vals1, 4 * Mc));
-    CHECKED(ctx->grow(ctx->hist, 4 * radix_hist_words((uint32_t)std::max(Mc, Nc))));
-    CHECKED(ctx->grow(ctx->slot_f, (Mc + 3) & ~(size_t)3));
-    // (tile << gbits) | id fits in 32 bits: the sort moves the keys alone
-    const int bits = tile_bits(ctx->ntiles);
-    int gbits = 1;
-    while (gbits < 31 && (1u << gbits) < (uint32_t)Nc) gbits++;
-    const bool packed = ctx->tuning.pack_keys && gbits + bits <= 32;
-    k.m_max = (uint32_t)M;
-    k.keys = (uint32_t *)ctx->keys0.p;
-    k.vals = packed ? nullptr : (int32_t *)ctx->vals0.p;
-    k.gid_bits = packed ? (uint32_t)gbits : 0u;
-    k.slot_f = (uint8_t *)ctx->slot_f.p;
-    launch_keygen_emit(k, false, s);
-    ctx->slot_f_clean = true;
-    uint32_t *kin = (uint32_t *)ctx->keys0.p, *kout = (uint32_t *)ctx->keys1.p;
-    int32_t *vin = packed ? nullptr : (int32_t *)ctx->vals0.p, *vout = packed ? nullptr : (int32_t *)ctx->vals1.p;
-    const int shift0 = packed ? gbits : 0;
-    // The first pass takes the bits left over by whole bytes (the last pass takes 8), so
-    // that it has fewer, longer digit runs: its input is in depth order, the least
-    // coalesced scatter of the sort.
-    for (int done = 0; done < bits;) {
-        const int width = done == 0 && bits % 8 ? bits % 8 : 8;
-        launch_radix_pass(kin, vin, kout, vout, ctx->d_total32(), (uint32_t)M, shift0 + done,
-                          (uint32_t *)ctx->hist.p, (uint32_t *)ctx->digit_total.p, s, (1u << width) - 1u);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
-        done += width;
-    }
-    ctx->keys_sorted = kin;
-    ctx->gid_sorted = vin;
-    ctx->sort_gid_bits = shift0;
-    launch_tile_ranges(kin, ctx->d_total32(), (uint32_t)M, nullptr, ctx->ntiles, (int32_t *)ctx->tile_start.p, s,
-                       shift0);
+    CHECKED(ctx->grow(ctx->coarse, 8 * Mc));
+    CHECKED(ctx->grow(ctx->gids, 4 * Mc));
+    t.coarse = (uint2 *)ctx->coarse.p;
+    t.gids = (int32_t *)ctx->gids.p;
+    launch_tile_lists_end(t, false, nodes, (uint32_t)V, (uint32_t)M, ntiles, part, s);
+    ctx->gid_sorted = t.gids;
     ctx->end();
     HIPCHECK(hipGetLastError());
     ctx->frame_stage = msplat_hip_ctx::FRAME_BINNED;
@@ -259,8 +219,7 @@ RasterArgs raster_args(msplat_hip_ctx *ctx) {
     r.tiles_x = ctx->tiles_x;
     r.tiles_y = ctx->tiles_y;
     r.tile_start = (const int32_t *)ctx->tile_start.p;
-    r.gid = ctx->sort_gid_bits ? (const int32_t *)ctx->keys_sorted : ctx->gid_sorted;
-    r.gid_mask = ctx->sort_gid_bits ? (1u << ctx->sort_gid_bits) - 1u : 0xFFFFFFFFu;
+    r.gid = ctx->gid_sorted;
     r.splat_a = (const float4 *)ctx->splat_a.p;
     r.splat_b = (const float4 *)ctx->splat_b.p;
     r.splat_blue = (const float *)ctx->splat_blue.p;
@@ -345,19 +304,21 @@ int do_raster_backward(msplat_hip_ctx *ctx) {
     CHECKED(ctx->grow(ctx->slot_c, 4 * Mc));
     CHECKED(ctx->grow(ctx->slot_f, (Mc + 3) & ~(size_t)3));
     if (ctx->frame_aux) CHECKED(ctx->grow(ctx->slot_d, 4 * Mc));
-    // the zero flags of the frame's slots: cleared by its key emission, or here when an
-    // earlier backward of the same frame has set some
-    if (!ctx->slot_f_clean) {
-        const size_t words = (Mc + 3) / 4;
-        zero_u32<<<(unsigned)std::min<size_t>((words + 255) / 256, 2048), 256, 0, ctx->stream>>>(
-            (uint32_t *)ctx->slot_f.p, words);
-    }
+    SlotPrepareArgs p;
+    p.flag_words = (uint32_t *)ctx->slot_f.p;
+    p.nwords = (Mc + 3) / 4;
+    p.count = (const uint32_t *)ctx->count.p;
+    p.nrec = ctx->big_listed ? 0u : (uint32_t)ctx->n;
+    p.overflow = ctx->capturing ? ctx->d_overflow() : nullptr;
+    p.big_list = ctx->big_list();
+    p.big_count = ctx->d_big_count();
+    launch_slot_prepare(p, ctx->stream);
+    ctx->big_listed = true;
     RasterArgs r = raster_args(ctx);
     r.slots_written = ctx->d_slots_written();
     ctx->begin(4);
     launch_raster_backward(r, ctx->tuning, ctx->stream);
     ctx->end();
-    ctx->slot_f_clean = false;
     HIPCHECK(hipGetLastError());
     return MSPLAT_OK;
 }
@@ -513,12 +474,9 @@ int frame_chunks_for(msplat_hip_ctx *ctx, int64_t m) {
 int capture_step(msplat_hip_ctx *ctx, const StepRecord &r) {
     drop_step_graph(ctx);
     // the capacity's buffers; every other one was sized by this shape's last eager step
-    const size_t Mc = (size_t)ctx->step_cap, N = (size_t)(r.g.num_points > 0 ? r.g.num_points : 1);
-    CHECKED(ctx->grow(ctx->keys0, 4 * Mc));
-    CHECKED(ctx->grow(ctx->keys1, 4 * Mc));
-    CHECKED(ctx->grow(ctx->vals0, 4 * Mc));
-    CHECKED(ctx->grow(ctx->vals1, 4 * Mc));
-    CHECKED(ctx->grow(ctx->hist, 4 * radix_hist_words((uint32_t)std::max(Mc, N))));
+    const size_t Mc = (size_t)ctx->step_cap;
+    CHECKED(ctx->grow(ctx->coarse, 8 * Mc));
+    CHECKED(ctx->grow(ctx->gids, 4 * Mc));
     CHECKED(ctx->grow(ctx->slot_f, (Mc + 3) & ~(size_t)3));
     CHECKED(ctx->grow(ctx->slot_a, 16 * Mc));
     CHECKED(ctx->grow(ctx->slot_b, 16 * Mc));
@@ -568,8 +526,7 @@ int capture_step(msplat_hip_ctx *ctx, const StepRecord &r) {
     ctx->step_gen = ctx->generation;
     ctx->step_captures++;
     ctx->step_frame = StepFrame{ctx->n,           ctx->width,      ctx->height,        ctx->tiles_x,
-                                ctx->tiles_y,     ctx->ntiles,     ctx->keys_sorted,   ctx->gid_sorted,
-                                ctx->sort_gid_bits, ctx->vis_sorted, ctx->frame_chunks, {ctx->bg[0], ctx->bg[1], ctx->bg[2]}};
+                                ctx->tiles_y,     ctx->ntiles,     ctx->gid_sorted,    ctx->vis_sorted, ctx->frame_chunks, {ctx->bg[0], ctx->bg[1], ctx->bg[2]}};
     return MSPLAT_OK;
 }
 
@@ -582,14 +539,12 @@ void restore_step_frame(msplat_hip_ctx *ctx) {
     ctx->tiles_x = f.tiles_x;
     ctx->tiles_y = f.tiles_y;
     ctx->ntiles = f.ntiles;
-    ctx->keys_sorted = f.keys_sorted;
     ctx->gid_sorted = f.gid_sorted;
-    ctx->sort_gid_bits = f.sort_gid_bits;
     ctx->vis_sorted = f.vis_sorted;
     ctx->frame_chunks = f.chunks;
     for (int i = 0; i < 3; i++) ctx->bg[i] = f.bg[i];
     ctx->frame_stage = msplat_hip_ctx::FRAME_RASTERED;
-    ctx->slot_f_clean = false;
+    ctx->big_listed = true;
     ctx->frame_aux = false;
 }
 
@@ -1163,19 +1118,10 @@ int msplat_hip_frame_view(msplat_hip_ctx *ctx, msplat_hip_frame *f) {
     f->offsets = (uint32_t *)ctx->offsets.p;
     f->isect_keys = nullptr;
     f->isect_gid = ctx->gid_sorted;
-    if ((ctx->flags & MSPLAT_FRAME_KEYS64) && ctx->keys_sorted) {
-        const uint32_t *tiles = ctx->keys_sorted;
-        if (ctx->sort_gid_bits) {  // split the packed keys into the key buffer not holding them, and vals0
-            uint32_t *spare = ctx->keys_sorted == (uint32_t *)ctx->keys0.p ? (uint32_t *)ctx->keys1.p
-                                                                           : (uint32_t *)ctx->keys0.p;
-            launch_unpack_keys(ctx->keys_sorted, (uint32_t)ctx->M, ctx->sort_gid_bits, spare,
-                               (int32_t *)ctx->vals0.p, ctx->stream);
-            tiles = spare;
-            f->isect_gid = (int32_t *)ctx->vals0.p;
-        }
+    if ((ctx->flags & MSPLAT_FRAME_KEYS64) && ctx->gid_sorted) {
         CHECKED(ctx->grow(ctx->keys64, 8 * (size_t)(ctx->M > 0 ? ctx->M : 1)));
-        launch_keys64(tiles, f->isect_gid, (const float *)ctx->depths.p, (uint32_t)ctx->M,
-                      (uint64_t *)ctx->keys64.p, ctx->stream);
+        launch_list_keys64((const int32_t *)ctx->tile_start.p, ctx->ntiles, ctx->gid_sorted,
+                           (const float *)ctx->depths.p, (uint64_t *)ctx->keys64.p, ctx->stream);
         HIPCHECK(hipGetLastError());
         f->isect_keys = (uint64_t *)ctx->keys64.p;
     }
@@ -1230,10 +1176,8 @@ int msplat_hip_radix_sort(msplat_hip_ctx *ctx, uint64_t *keys, int32_t *vals, ui
         HIPCHECK(hipMemcpyAsync(vals, vin, 4 * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
     }
     HIPCHECK(hipGetLastError());
-    // the frame's sorted intersections lived in keys1/vals1; they are no longer valid
-    ctx->keys_sorted = nullptr;
+    // the call ends the frame in the workspace: its lists are no longer offered
     ctx->gid_sorted = nullptr;
-    ctx->sort_gid_bits = 0;
     if (ctx->frame_stage > msplat_hip_ctx::FRAME_PROJECTED) ctx->frame_stage = msplat_hip_ctx::FRAME_PROJECTED;
     return MSPLAT_OK;
 }

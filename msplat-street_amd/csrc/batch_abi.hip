@@ -21,10 +21,10 @@ namespace msplat {
 struct BatchState {
     // per record (views x gaussians)
     Buf splat_a, splat_b, splat_blue, depths, rect, radii, count, offsets, block_sums, block_vis, big_list, big_sums;
-    // visible records sorted by depth, count sums in depth order, scan partials
-    Buf dk0, dk1, dv0, dv1, ord_sums, scan_part, loff;
+    // visible records sorted by depth, radix and scan partials, tile list scratch
+    Buf dk0, dk1, dv0, dv1, hist, digit_total, scan_part, lrect, lists;
     // per intersection
-    Buf keys0, keys1, vals0, vals1, slot_a, slot_b, slot_c, slot_f, hist, digit_total;
+    Buf coarse, gids, slot_a, slot_b, slot_c, slot_f;
     // per tile, pixel, row
     Buf tile_start, image, final_T, final_idx, v_image, row_loss, loss_scratch;
     // summed gradients (per gaussian), visibility in any view
@@ -36,12 +36,12 @@ struct BatchState {
     bool tab_pending = false;
     uint32_t cap = 0;  // intersection capacity
     uint32_t tiles_cap = 0, pixels_cap = 0, rows_cap = 0, loss_cap = 0;
-    uint32_t vtiles_cap = 0;  // tiles of the largest view (the local tile sort's key range)
+    uint32_t nodes_cap = 0;  // level-1 nodes of the tile lists
     int n = 0, views = 0;
     uint64_t generation = 0;  // bumped when a buffer moves
     // the last rendered frame
     bool rendered = false;
-    bool slot_f_clean = false;  // slot_f of the last frame is all zero (its key emission ran, no backward yet)
+    bool big_listed = false;  // the last frame's list of records with many intersections is built
     int frame_n = 0;
     uint32_t frame_w[MAX_VIEWS] = {}, frame_h[MAX_VIEWS] = {};
     int32_t *gid_sorted = nullptr;
@@ -55,10 +55,10 @@ struct BatchState {
 
 void destroy_batch_state(BatchState *b) {
     if (!b) return;
-    Buf *all[] = {&b->loff, &b->block_vis, &b->dk0, &b->dk1, &b->dv0, &b->dv1, &b->ord_sums, &b->scan_part,
+    Buf *all[] = {&b->lrect, &b->lists, &b->block_vis, &b->dk0, &b->dk1, &b->dv0, &b->dv1, &b->scan_part,
                   &b->splat_a, &b->splat_b, &b->splat_blue, &b->depths,   &b->rect,     &b->radii,      &b->count,
-                  &b->offsets, &b->block_sums, &b->big_list, &b->big_sums, &b->keys0, &b->keys1,    &b->vals0,
-                  &b->vals1,   &b->slot_a,     &b->slot_b,   &b->slot_c,   &b->slot_f, &b->hist,  &b->digit_total, &b->tile_start,
+                  &b->offsets, &b->block_sums, &b->big_list, &b->big_sums, &b->coarse, &b->gids,
+                  &b->slot_a,     &b->slot_b,   &b->slot_c,   &b->slot_f, &b->hist,  &b->digit_total, &b->tile_start,
                   &b->image,   &b->final_T,    &b->final_idx, &b->v_image, &b->row_loss, &b->loss_scratch, &b->grads,
                   &b->vis_any, &b->table,      &b->scalars};
     for (Buf *x : all)
@@ -100,17 +100,8 @@ int grow(msplat_hip_ctx *ctx, BatchState *b, Buf &buf, size_t bytes) {
 
 size_t record_count(BatchState *b) { return (size_t)b->views * (size_t)(b->n > 0 ? b->n : 1); }
 
-// Radix histograms for the larger of the two sorts: the depth sort over every record
-// and the tile sort over the intersection capacity.
-int grow_sort_scratch(msplat_hip_ctx *ctx, BatchState *b) {
-    const size_t n = std::max((size_t)b->cap, record_count(b));
-    CHECKED(grow(ctx, b, b->hist, 4 * radix_hist_words((uint32_t)n)));
-    CHECKED(grow(ctx, b, b->digit_total, 4 * 256));
-    return MSPLAT_OK;
-}
-
 struct Layout {
-    uint32_t tiles = 0, pixels = 0, rows = 0, loss_blocks = 0;
+    uint32_t tiles = 0, pixels = 0, rows = 0, loss_blocks = 0, nodes = 0;
 };
 
 int check_views(const msplat_hip_gaussians *g, const msplat_hip_views *views, bool training) {
@@ -157,6 +148,8 @@ int prepare(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g, c
         t.tile_base[v] = L.tiles;
         t.row_base[v] = L.rows;
         t.loss_base[v] = L.loss_blocks;
+        t.node_base[v] = L.nodes;
+        L.nodes += tile_list_nodes(c.tiles_x, c.tiles_y);
         const uint64_t pix = (uint64_t)L.pixels + (uint64_t)c.width * c.height;
         if (pix > 0x7FFFFFFFull) return set_error(MSPLAT_ERR_RANGE, "the batch exceeds 2^31 pixels");
         L.pixels = (uint32_t)pix;
@@ -165,10 +158,7 @@ int prepare(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g, c
         L.loss_blocks += loss_blocks(c.width, c.height);
     }
     t.tile_base[nv] = L.tiles;
-    uint32_t vt = 1;
-    for (int v = 0; v < nv; v++)
-        vt = std::max(vt, (uint32_t)(views->cameras[v].tiles_x * views->cameras[v].tiles_y));
-    t.max_view_tiles = vt;
+    t.node_base[nv] = L.nodes;
     t.row_base[nv] = L.rows;
     t.loss_base[nv] = L.loss_blocks;
     t.total_tiles = L.tiles;
@@ -205,17 +195,20 @@ int prepare(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g, c
     CHECKED(grow(ctx, b, b->dk1, 4 * R));
     CHECKED(grow(ctx, b, b->dv0, 4 * R));
     CHECKED(grow(ctx, b, b->dv1, 4 * R));
-    CHECKED(grow(ctx, b, b->loff, 4 * R));
-    CHECKED(grow(ctx, b, b->ord_sums, 4 * ((R + 255) / 256 + 1)));
-    CHECKED(grow(ctx, b, b->scan_part, 4 * 3 * scan_partial_words((uint32_t)std::max(nbx * nv, (R + 255) / 256)) + 64));
+    CHECKED(grow(ctx, b, b->lrect, 8 * R));
+    CHECKED(grow(ctx, b, b->hist, 4 * radix_hist_words((uint32_t)R)));
+    CHECKED(grow(ctx, b, b->digit_total, 4 * 256));
     CHECKED(grow(ctx, b, b->big_list, 4 * R));
     CHECKED(grow(ctx, b, b->big_sums, 36 * R + 64));
-    b->tiles_cap = std::max(b->tiles_cap, std::max(L.tiles, vt * (uint32_t)nv));  // items and ranges
-    b->vtiles_cap = std::max(b->vtiles_cap, vt);
+    b->tiles_cap = std::max(b->tiles_cap, L.tiles);
+    b->nodes_cap = std::max(b->nodes_cap, L.nodes);
     b->pixels_cap = std::max(b->pixels_cap, L.pixels);
     b->rows_cap = std::max(b->rows_cap, L.rows);
     b->loss_cap = std::max(b->loss_cap, L.loss_blocks);
     CHECKED(grow(ctx, b, b->tile_start, 4 * ((size_t)b->tiles_cap + 1)));
+    CHECKED(grow(ctx, b, b->lists, 4 * tile_list_scratch_words(b->nodes_cap)));
+    CHECKED(grow(ctx, b, b->scan_part,
+                 4 * 2 * scan_partial_words((uint32_t)std::max<size_t>(nbx * nv, (size_t)b->tiles_cap + 1)) + 64));
     const size_t P = b->pixels_cap > 0 ? b->pixels_cap : 1;
     CHECKED(grow(ctx, b, b->image, 12 * P));
     CHECKED(grow(ctx, b, b->final_T, 4 * P));
@@ -227,7 +220,6 @@ int prepare(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g, c
     CHECKED(grow(ctx, b, b->scalars, sizeof(BatchScalars)));
     b->n = n;
     b->views = nv;
-    CHECKED(grow_sort_scratch(ctx, b));  // the record count may have grown
     (void)batch_raster_grid(false, ctx->tuning);  // occupancy queries outside any capture
     (void)batch_raster_grid(true, ctx->tuning);
     HIPCHECK(hipMemcpyAsync(b->table.p, b->h_tab, sizeof(BatchTable), hipMemcpyHostToDevice, ctx->stream));
@@ -243,16 +235,14 @@ int grow_isects(msplat_hip_ctx *ctx, BatchState *b, uint64_t need) {
                          (unsigned long long)need);
     if (want <= b->cap && b->cap) return MSPLAT_OK;
     const size_t C = (size_t)want;
-    CHECKED(grow(ctx, b, b->keys0, 4 * C));
-    CHECKED(grow(ctx, b, b->keys1, 4 * C));
-    CHECKED(grow(ctx, b, b->vals0, 4 * C));
-    CHECKED(grow(ctx, b, b->vals1, 4 * C));
+    CHECKED(grow(ctx, b, b->coarse, 8 * C));
+    CHECKED(grow(ctx, b, b->gids, 4 * C));
     CHECKED(grow(ctx, b, b->slot_a, 16 * C));
     CHECKED(grow(ctx, b, b->slot_b, 16 * C));
     CHECKED(grow(ctx, b, b->slot_c, 4 * C));
     CHECKED(grow(ctx, b, b->slot_f, (C + 3) & ~(uint64_t)3));
     b->cap = (uint32_t)C;
-    return grow_sort_scratch(ctx, b);
+    return MSPLAT_OK;
 }
 
 BatchScalars *dsc(BatchState *b) { return (BatchScalars *)b->scalars.p; }
@@ -316,7 +306,7 @@ float4 *big_a(BatchState *b) { return (float4 *)(((uintptr_t)b->big_sums.p + 15)
 
 uint32_t *scan_parts(BatchState *b, int i) {
     const size_t pw = scan_partial_words((uint32_t)std::max((size_t)b->views * ((b->n + 255) / 256),
-                                                            (record_count(b) + 255) / 256));
+                                                            (size_t)b->tiles_cap + 1));
     return (uint32_t *)b->scan_part.p + i * pw;
 }
 
@@ -332,7 +322,7 @@ void enqueue_counts(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussia
                     ScanOut{&sc->nvis64, &sc->nvis, 0xFFFFFFFFu, nullptr, nullptr}, s);
 }
 
-// visible records sorted by depth, keys in depth order, tile sort, ranges, forward
+// visible records sorted by depth, the tiles' lists, forward
 void enqueue_sort_and_forward(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g) {
     hipStream_t s = ctx->stream;
     BatchScalars *sc = dsc(b);
@@ -344,6 +334,8 @@ void enqueue_sort_and_forward(msplat_hip_ctx *ctx, BatchState *b, const msplat_h
     c.count = (const uint32_t *)b->count.p;
     c.depths = (const float *)b->depths.p;
     c.block_vis = (const uint32_t *)b->block_vis.p;
+    c.block_sums = (const uint32_t *)b->block_sums.p;
+    c.offsets = (uint32_t *)b->offsets.p;
     c.dkeys = (uint32_t *)b->dk0.p;
     c.dvals = (int32_t *)b->dv0.p;
     launch_compact(c, s);
@@ -360,57 +352,41 @@ void enqueue_sort_and_forward(msplat_hip_ctx *ctx, BatchState *b, const msplat_h
     launch_radix_pass(dki, dvi, dko, dvo, &sc->nvis, R, 0, (uint32_t *)b->hist.p, (uint32_t *)b->digit_total.p, s);
     std::swap(dki, dko);
     std::swap(dvi, dvo);
-    launch_order_sums(dvi, &sc->nvis, R, (const uint32_t *)b->count.p, (uint32_t *)b->ord_sums.p,
-                      (uint32_t *)b->loff.p, s);
-    launch_scan_u32((uint32_t *)b->ord_sums.p, (R + 255) / 256, scan_parts(b, 2),
-                    ScanOut{nullptr, &sc->total32_b, b->cap, &sc->overflow_b, nullptr}, s);
-    KeygenArgs k;
-    memset(&k, 0, sizeof k);
-    k.list = dvi;
-    k.nvis_ptr = &sc->nvis;
-    k.nvis_max = R;
-    k.count = (const uint32_t *)b->count.p;
-    k.rect = (const uint2 *)b->rect.p;
-    k.block_bases = (const uint32_t *)b->ord_sums.p;
-    k.offsets = (uint32_t *)b->offsets.p;
-    k.loff = (uint32_t *)b->loff.p;
-    k.m_ptr = &sc->total32;
-    k.m_max = b->cap;
-    k.keys = (uint32_t *)b->keys0.p;
-    k.vals = (int32_t *)b->vals0.p;
-    k.big_list = (uint32_t *)b->big_list.p;
-    k.big_count = &sc->big_count;
-    k.overflow = &sc->overflow;
-    k.tab = dtab(b);
-    k.n = g->num_points;
-    k.slot_f = (uint8_t *)b->slot_f.p;
-    launch_keygen(k, true, s);
-    uint32_t *kin = (uint32_t *)b->keys0.p, *kout = (uint32_t *)b->keys1.p;
-    int32_t *vin = (int32_t *)b->vals0.p, *vout = (int32_t *)b->vals1.p;
-    const int bits = tile_bits((int)b->vtiles_cap);
-    for (int done = 0; done < bits;) {  // narrow first pass, as for one view (abi.hip)
-        const int width = done == 0 && bits % 8 ? bits % 8 : 8;
-        launch_radix_pass(kin, vin, kout, vout, &sc->total32, b->cap, done, (uint32_t *)b->hist.p,
-                          (uint32_t *)b->digit_total.p, s, (1u << width) - 1u);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
-        done += width;
-    }
-    b->gid_sorted = vin;
-    launch_tile_ranges_views(kin, vin, &sc->total32, b->cap, g->num_points, dtab(b), (int32_t *)b->tile_start.p, s);
+    TileListArgs t;
+    memset(&t, 0, sizeof t);
+    t.list = dvi;
+    t.nvis = &sc->nvis;
+    t.overflow = &sc->overflow;
+    t.rect = (const uint2 *)b->rect.p;
+    t.lrect = (uint2 *)b->lrect.p;
+    t.coarse = (uint2 *)b->coarse.p;
+    t.gids = (int32_t *)b->gids.p;
+    t.tile_start = (int32_t *)b->tile_start.p;
+    t.tab = dtab(b);
+    t.block_vis = (const uint32_t *)b->block_vis.p;
+    t.nbx = (g->num_points + 255) / 256;
+    tile_list_carve((uint32_t *)b->lists.p, b->nodes_cap, t);
+    launch_tile_lists_begin(t, true, b->nodes_cap, R, s);
+    launch_tile_lists_end(t, true, b->nodes_cap, R, b->cap, b->tiles_cap, scan_parts(b, 0), s);
+    b->gid_sorted = t.gids;
+    b->big_listed = false;
     launch_batch_raster_forward(raster_args(b), ctx->tuning, s);
 }
 
-// raster backward, big-list sums, per-gaussian sums over the views. The slots' zero flags
-// are all zero after the frame's key emission; a later backward of the same frame
-// (clear_flags) zeroes them first.
+// the slots' zero flags cleared and the big list built, raster backward, big-list sums, per-gaussian sums over the views
 void enqueue_backward(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussians *g, float *const gout[6],
-                      const msplat_hip_grad_stats *stats, bool clear_flags) {
+                      const msplat_hip_grad_stats *stats) {
     hipStream_t s = ctx->stream;
-    if (clear_flags) {
-        const size_t words = (b->cap + 3) / 4;
-        if (words) zero_u32<<<(unsigned)std::min<size_t>((words + 255) / 256, 2048), 256, 0, s>>>((uint32_t *)b->slot_f.p, words);
-    }
+    SlotPrepareArgs p;
+    p.flag_words = (uint32_t *)b->slot_f.p;
+    p.nwords = ((size_t)b->cap + 3) / 4;
+    p.count = (const uint32_t *)b->count.p;
+    p.nrec = b->big_listed ? 0u : (uint32_t)((size_t)b->views * (size_t)g->num_points);
+    p.overflow = &dsc(b)->overflow;
+    p.big_list = (uint32_t *)b->big_list.p;
+    p.big_count = &dsc(b)->big_count;
+    launch_slot_prepare(p, s);
+    b->big_listed = true;
     launch_batch_raster_backward(raster_args(b), ctx->tuning, s);
     const size_t R = record_count(b);
     float4 *ba = big_a(b);
@@ -484,7 +460,7 @@ void enqueue_train(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gaussian
     l.row_loss = (double *)b->row_loss.p;
     l.sc = dsc(b);
     launch_batch_loss(l, s);
-    enqueue_backward(ctx, b, g, gr, stats, false);
+    enqueue_backward(ctx, b, g, gr, stats);
     const size_t N = (size_t)g->num_points;
     const uint32_t stride = (sh_bases(b->h_tab->views[0].cam.degree) - 1) * 3;
     float *params[6] = {g->means, g->scales, g->quats, g->features_dc, g->features_rest, g->opacities};
@@ -539,7 +515,7 @@ std::vector<uint64_t> graph_key(msplat_hip_ctx *ctx, BatchState *b, const msplat
                                 const msplat_hip_adam *adam, const msplat_hip_grad_stats *st) {
     std::vector<uint64_t> k = {(uint64_t)b->n,          (uint64_t)b->views,       b->cap,
                                b->tiles_cap,            b->pixels_cap,            b->rows_cap,
-                               b->loss_cap,             b->generation,            b->vtiles_cap,            (uint64_t)ctx->tuning.bwd_ppt,
+                               b->loss_cap,             b->generation,            b->nodes_cap,             (uint64_t)ctx->tuning.bwd_ppt,
                                (uint64_t)ctx->tuning.fwd_batch, (uint64_t)ctx->tuning.bwd_batch,
                                (uint64_t)ctx->tuning.cull,
                                b->h_tab->views[0].cam.degree};
@@ -611,7 +587,6 @@ int msplat_hip_render_batch(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, 
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     b->rendered = true;
-    b->slot_f_clean = true;
     b->frame_n = g->num_points;
     for (int v = 0; v < views->num_views; v++) {
         b->frame_w[v] = views->cameras[v].width;
@@ -668,8 +643,7 @@ int msplat_hip_render_backward_batch(msplat_hip_ctx *ctx, const msplat_hip_gauss
                       out->v_opacities};
     float *gr[6];
     for (int i = 0; i < 6; i++) gr[i] = user[i] ? user[i] : scratch[i];
-    enqueue_backward(ctx, b, g, gr, nullptr, !b->slot_f_clean);
-    b->slot_f_clean = false;
+    enqueue_backward(ctx, b, g, gr, nullptr);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     return MSPLAT_OK;

@@ -1,5 +1,5 @@
-// Projection + SH colour, binning of the splats into 16x16 tiles, stable LSD radix
-// sort and per-tile range extraction.
+// Projection + SH colour, the visible records' depth order, and the stable LSD radix
+// sort.
 //
 // Layout in HBM (per record, SoA, written once per view; a record is a gaussian in one
 // view, record v * n + g in a batch of views):
@@ -8,14 +8,10 @@
 //   splat_blue = b, depths, aabb (float2), rect (x0 | x1 << 16, y0 | y1 << 16), count
 //
 // Binning keeps the reference's per-tile order, ascending (depth bits, gaussian id)
-// (core/cpu/msplat_cpu.cpp:505-537), with two small stable sorts in place of one sort
-// of 64-bit (tile | depth) keys:
-//   1. the visible records are compacted in id order and stably sorted by their 32-bit
-//      depth bits (4 passes over the visible records, not over the intersections);
-//   2. each record's intersections are emitted in that depth order with its tile id as
-//      a 32-bit key, and a stable sort by tile (ceil(tile bits / 8) passes) leaves every
-//      tile's intersections in (depth, id) order.
-// Records own contiguous slot ranges (offsets[r], count[r]) in emission order, tiles
+// (core/cpu/msplat_cpu.cpp:505-537): the visible records are compacted in id order and
+// stably sorted by their 32-bit depth bits (4 passes over the visible records, not over
+// the intersections), and the tiles' lists are expanded from that order (tile_lists.hip).
+// Records own contiguous slot ranges (offsets[r], count[r]) in record order, tiles
 // row-major within a record, which the backward's per-record reductions read.
 #include <algorithm>
 
@@ -219,33 +215,63 @@ __global__ __launch_bounds__(256) void scan_top_kernel(uint32_t *partial, int nc
     }
 }
 
-// The whole scan in one workgroup, 4096 entries at a time (small arrays)
+// The whole scan in one workgroup of 1024 threads, 16384 entries at a time: one launch and
+// one round for up to 4M gaussians' block sums or a 2560x1440 view's tiles.
+constexpr int SCAN_SMALL_THREADS = 1024, SCAN_SMALL_CHUNK = 16 * SCAN_SMALL_THREADS;
 __device__ inline void scan_small(uint32_t *a, uint32_t L, const ScanOut &o) {
-    __shared__ uint32_t lds4[4];
-    __shared__ uint64_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (uint32_t chunk = 0; chunk < L; chunk += SCAN_CHUNK) {
+    __shared__ uint32_t wsum[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint64_t carry = 0;  // the same in every thread
+    const bool wide = ((uintptr_t)a & 15) == 0;  // a thread's 16 entries as four 16-byte loads and stores
+    for (uint32_t chunk = 0; chunk < L; chunk += SCAN_SMALL_CHUNK) {
         const uint32_t base = chunk + threadIdx.x * 16;
+        const bool whole = wide && base + 16 <= L;
         uint32_t v[16], sum = 0;
+        if (whole) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint4 q = ((const uint4 *)(a + base))[i];
+                v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = base + i < L ? a[base + i] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) sum += v[i];
+        uint32_t x = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d);
+            if (lane >= d) x += y;
+        }
+        if (lane == 63) wsum[w] = x;
+        __syncthreads();
+        uint32_t pre = 0, total = 0;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            v[i] = base + i < L ? a[base + i] : 0u;
-            sum += v[i];
+            const uint32_t t = wsum[i];
+            pre += i < w ? t : 0u;
+            total += t;
         }
-        uint32_t t;
-        const uint32_t ex = block_scan_u32(sum, t, lds4);
-        const uint64_t c = carry;
-        uint32_t run = (uint32_t)c + ex;
+        __syncthreads();  // wsum is written again
+        uint32_t run = (uint32_t)carry + pre + x - sum;
 #pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (base + i < L) {
-                a[base + i] = run;
-                run += v[i];
-            }
-        __syncthreads();
-        if (threadIdx.x == 0) carry = c + t;
-        __syncthreads();
+        for (int i = 0; i < 16; i++) {
+            const uint32_t t = v[i];
+            v[i] = run;
+            run += t;
+        }
+        if (whole) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                ((uint4 *)(a + base))[i] = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (base + i < L) a[base + i] = v[i];
+        }
+        carry += total;
     }
     if (threadIdx.x == 0) {
         const uint64_t tot = carry;
@@ -259,11 +285,13 @@ __device__ inline void scan_small(uint32_t *a, uint32_t L, const ScanOut &o) {
     }
 }
 
-__global__ __launch_bounds__(256) void scan_small_kernel(uint32_t *a, uint32_t L, ScanOut o) { scan_small(a, L, o); }
+__global__ __launch_bounds__(SCAN_SMALL_THREADS) void scan_small_kernel(uint32_t *a, uint32_t L, ScanOut o) {
+    scan_small(a, L, o);
+}
 
 // Two small scans of the same length in one launch, one workgroup each
-__global__ __launch_bounds__(256) void scan_small_pair_kernel(uint32_t *a0, ScanOut o0, uint32_t *a1, ScanOut o1,
-                                                              uint32_t L) {
+__global__ __launch_bounds__(SCAN_SMALL_THREADS) void scan_small_pair_kernel(uint32_t *a0, ScanOut o0, uint32_t *a1,
+                                                                            ScanOut o1, uint32_t L) {
     if (blockIdx.x == 0) scan_small(a0, L, o0);
     else scan_small(a1, L, o1);
 }
@@ -288,19 +316,51 @@ __global__ __launch_bounds__(256) void scan_apply_kernel(uint32_t *a, uint32_t L
 }
 
 // ── visible records in id order, keyed by depth bits ──────────────────────────
+// Also each record's intersection offset (the slots of the raster backward lie in record
+// order).
 __global__ __launch_bounds__(256) void compact_kernel(CompactArgs a) {
     __shared__ uint32_t lds4[4];
     const int v = blockIdx.y;
     const int g = blockIdx.x * 256 + threadIdx.x;
     const size_t r = (size_t)v * a.n + g;
-    const bool vis = g < a.n && a.count[r] > 0;
+    const uint32_t c = g < a.n ? a.count[r] : 0u;
+    const bool vis = c > 0;
     uint32_t t;
     const uint32_t ex = block_scan_u32(vis ? 1u : 0u, t, lds4);
+    if (t == 0) return;  // uniform: nothing visible in this workgroup
+    const uint32_t off = block_scan_u32(c, t, lds4);
     if (vis) {
-        const uint32_t pos = a.block_vis[(size_t)v * a.nbx + blockIdx.x] + ex;
+        const size_t blk = (size_t)v * a.nbx + blockIdx.x;
+        const uint32_t pos = a.block_vis[blk] + ex;
         a.dkeys[pos] = __float_as_uint(a.depths[r]);
         a.dvals[pos] = (int32_t)r;
+        a.offsets[r] = a.block_sums[blk] + off;
     }
+}
+
+// Clears the slots' zero flags and lists the records with more than BIG_SLOTS
+// intersections (in no particular order): each workgroup counts those of its part of the
+// records, takes its place in the list with one atomic, and writes them. One atomic per
+// 256 records, as the list was first built, serialised on its counter (about 12 ns each:
+// 21 us at 475k records, 360 us for a batch of 8 views of 1M).
+constexpr int SLOT_PREPARE_GRID = 1024;
+__global__ __launch_bounds__(256) void slot_prepare_kernel(SlotPrepareArgs a) {
+    __shared__ uint32_t lds4[4];
+    __shared__ uint32_t s_base;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < a.nwords; i += (size_t)gridDim.x * 256) a.flag_words[i] = 0u;
+    if (a.overflow && *a.overflow) return;
+    const uint32_t per = (a.nrec + gridDim.x - 1) / gridDim.x;
+    const uint32_t b = min(blockIdx.x * per, a.nrec), e = min(b + per, a.nrec);
+    uint32_t n = 0;
+    for (uint32_t r = b + threadIdx.x; r < e; r += 256) n += a.count[r] > BIG_SLOTS ? 1u : 0u;
+    uint32_t total;
+    uint32_t p = block_scan_u32(n, total, lds4);
+    if (total == 0) return;
+    if (threadIdx.x == 0) s_base = atomicAdd(a.big_count, total);
+    __syncthreads();
+    p += s_base;
+    for (uint32_t r = b + threadIdx.x; r < e; r += 256)
+        if (a.count[r] > BIG_SLOTS) a.big_list[p++] = r;
 }
 
 // ── stable LSD radix sort, 8-bit digits, 32- or 64-bit keys, int32 payload ─────
@@ -469,256 +529,12 @@ __global__ __launch_bounds__(256) void rs_scatter_kernel(const K *kin, const int
     }
 }
 
-// ── intersections in depth order ──────────────────────────────────────────────
-
-// Per 256-entry block of the depth-ordered list: the sum of its records' counts
-// (0 for blocks past the list's device-side length). Each record's count also goes to
-// lcount[i] in list order, so the offsets kernel reads it without a second gather.
-__global__ __launch_bounds__(256) void order_sums_kernel(const int32_t *list, const uint32_t *nvis_ptr,
-                                                        const uint32_t *count, uint32_t *sums, uint32_t nchunks_max,
-                                                        uint32_t *lcount) {
-    __shared__ uint32_t lds4[4];
-    const uint32_t nvis = *nvis_ptr;
-    for (uint32_t chunk = blockIdx.x; chunk < nchunks_max; chunk += gridDim.x) {
-        if (chunk * 256 >= nvis) {  // past the list: zero sums, nothing to read
-            if (threadIdx.x == 0) sums[chunk] = 0;
-            continue;
-        }
-        const uint32_t i = chunk * 256 + threadIdx.x;
-        const uint32_t c = i < nvis ? count[list[i]] : 0u;
-        if (i < nvis) lcount[i] = c;
-        uint32_t t;
-        block_scan_u32(c, t, lds4);
-        if (threadIdx.x == 0) sums[chunk] = t;
-    }
-}
-
-// Record list[i] writes its tiles in row-major order at offsets[r] = the exclusive
-// prefix of the counts in list order (also kept in list order, loff[i], for the
-// emission), and joins the big list when it has more than BIG_SLOTS intersections.
-// loff[i] holds the record's count on entry (order_sums_kernel).
-__global__ __launch_bounds__(256) void keygen_offsets_kernel(KeygenArgs a) {
-    __shared__ uint32_t lds4[4];
-    __shared__ uint32_t s_bigbase;
-    if (a.overflow && *a.overflow) return;
-    const uint32_t nvis = *a.nvis_ptr;
-    for (uint32_t chunk = blockIdx.x; chunk * 256 < nvis; chunk += gridDim.x) {
-        const uint32_t i = chunk * 256 + threadIdx.x;
-        const int32_t r = i < nvis ? a.list[i] : -1;
-        const uint32_t c = r >= 0 ? a.loff[i] : 0u;
-        uint32_t total;
-        uint32_t base;
-        if (a.chunk_sums) {  // the sums of the chunks before this one, added here
-            uint32_t part = 0;
-            for (uint32_t q = threadIdx.x; q < chunk; q += 256) part += a.chunk_sums[q];
-            block_scan_u32(part, base, lds4);
-        } else {
-            base = a.block_bases[chunk];
-        }
-        const uint32_t off = base + block_scan_u32(c, total, lds4);
-        if (r >= 0) {
-            a.offsets[r] = off;
-            a.loff[i] = off;
-        }
-        uint32_t nbig;
-        const uint32_t bex = block_scan_u32(c > BIG_SLOTS ? 1u : 0u, nbig, lds4);
-        if (threadIdx.x == 0 && nbig) s_bigbase = atomicAdd(a.big_count, nbig);
-        __syncthreads();
-        if (c > BIG_SLOTS) a.big_list[s_bigbase + bex] = (uint32_t)r;
-        __syncthreads();
-    }
-}
-
-// Key emission balanced over the output: workgroup b writes intersections
-// [b * EMIT_CHUNK, (b + 1) * EMIT_CHUNK). It finds the records covering its slice by a
-// block search over loff and stages their offsets, ids and tile rectangles in LDS, marking
-// where each record after the first starts. Thread t then writes the slice's outputs
-// 8t..8t+7: the record of output p is the number of marks at or before p (a block scan of
-// the threads' mark counts), and its tile follows from the previous output's by one step
-// along the rectangle's row, so one division per thread places its first output. The eight
-// keys (and ids) go out as two 16-byte stores; consecutive threads write consecutive
-// keys whatever the records' footprints (depth order puts the large near splats next to
-// each other).
-constexpr int EMIT_ITEMS = 8;
-constexpr int EMIT_CHUNK = 256 * EMIT_ITEMS;
-
-template <bool BATCH>
-__global__ __launch_bounds__(256) void keygen_emit_kernel(KeygenArgs a) {
-    __shared__ uint32_t s_off[EMIT_CHUNK];
-    __shared__ int32_t s_rec[EMIT_CHUNK];
-    __shared__ uint2 s_rect[EMIT_CHUNK];
-    __shared__ __align__(8) uint8_t s_mark[EMIT_CHUNK];
-    __shared__ uint32_t s_first, s_n;
-    __shared__ uint32_t lds4[4];
-    if (a.overflow && *a.overflow) return;
-    const uint32_t M = *a.m_ptr;
-    const uint32_t o0 = blockIdx.x * EMIT_CHUNK;
-    if (o0 >= M) return;
-    const uint32_t o1 = min(o0 + (uint32_t)EMIT_CHUNK, M);
-    {
-        // records first..last cover [o0, o1): the last i with loff[i] <= o0, o1 - 1 (loff
-        // rises from loff[0] = 0). A 256-ary search: each round every thread tests one
-        // probe of each range, and the count of probes at or below the target narrows
-        // the range [lo, hi) 256-fold (3 rounds for 3M records, every thread in step).
-        const uint32_t nvis = *a.nvis_ptr;
-        uint32_t lo1 = 0, hi1 = nvis, lo2 = 0, hi2 = nvis;
-        while (hi1 - lo1 > 1 || hi2 - lo2 > 1) {
-            const uint32_t st1 = (hi1 - lo1 + 255) / 256, st2 = (hi2 - lo2 + 255) / 256;
-            const uint32_t i1 = lo1 + threadIdx.x * st1, i2 = lo2 + threadIdx.x * st2;
-            const int c1 = __syncthreads_count(i1 < hi1 && a.loff[i1] <= o0);
-            const int c2 = __syncthreads_count(i2 < hi2 && a.loff[i2] <= o1 - 1);
-            lo1 += (uint32_t)(c1 - 1) * st1;
-            hi1 = min(lo1 + st1, hi1);
-            lo2 += (uint32_t)(c2 - 1) * st2;
-            hi2 = min(lo2 + st2, hi2);
-        }
-        if (threadIdx.x == 0) {
-            s_first = lo1;
-            s_n = lo2 - lo1 + 1;  // <= o1 - o0: every record after the first starts inside the slice
-        }
-        ((uint32_t *)s_mark)[threadIdx.x] = 0u;
-        ((uint32_t *)s_mark)[threadIdx.x + 256] = 0u;
-    }
-    __syncthreads();
-    const uint32_t first = s_first, nrec = s_n;
-    for (uint32_t j = threadIdx.x; j < nrec; j += 256) {
-        const uint32_t off = a.loff[first + j];
-        const int32_t rec = a.list[first + j];
-        s_off[j] = off;
-        s_rec[j] = rec;
-        s_rect[j] = a.rect[rec];
-        if (j > 0) s_mark[off - o0] = 1;  // in (0, o1 - o0): records after the first start inside
-    }
-    __syncthreads();
-    const uint32_t p0 = EMIT_ITEMS * threadIdx.x;
-    const uint2 mk = *(const uint2 *)(s_mark + p0);
-    uint32_t m[EMIT_ITEMS];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        m[i] = (mk.x >> (8 * i)) & 0xFFu;
-        m[4 + i] = (mk.y >> (8 * i)) & 0xFFu;
-    }
-    uint32_t total;
-    uint32_t j = block_scan_u32(m[0] + m[1] + m[2] + m[3] + m[4] + m[5] + m[6] + m[7], total, lds4);
-    if (o0 + p0 >= o1) return;
-    uint32_t kv[EMIT_ITEMS], vv[EMIT_ITEMS];
-    uint32_t q = 0, rem = 0, w = 1, x0 = 0, y0 = 0, tiles_x = (uint32_t)a.tiles_x;
-    int32_t r = 0;
-#pragma unroll
-    for (int i = 0; i < EMIT_ITEMS; i++) {
-        const bool start = m[i] != 0u;  // record j + 1 starts at this output
-        j += m[i];
-        if (i == 0 || start) {
-            r = s_rec[j];
-            const uint2 rr = s_rect[j];
-            x0 = rr.x & 0xFFFF;
-            w = (rr.x >> 16) - x0;
-            y0 = rr.y & 0xFFFF;
-            const uint32_t local = o0 + p0 + (uint32_t)i - s_off[j];
-            q = local / w;
-            rem = local - q * w;
-            // local tile id (a batch keeps its views apart by the emission order)
-            if (BATCH) tiles_x = (uint32_t)a.tab->views[r / a.n].cam.tiles_x;
-        } else if (++rem == w) {
-            rem = 0;
-            q++;
-        }
-        const uint32_t tile = (y0 + q) * tiles_x + (x0 + rem);
-        if (!BATCH && a.gid_bits) {
-            kv[i] = (tile << a.gid_bits) | (uint32_t)r;
-        } else {
-            kv[i] = tile;
-            vv[i] = (uint32_t)r;
-        }
-    }
-    const bool vals = BATCH || !a.gid_bits;
-    const uint32_t ob = o0 + p0;
-    if (ob + EMIT_ITEMS <= o1) {  // 32-byte aligned: o0 is a multiple of EMIT_CHUNK
-        uint4 *kd = (uint4 *)(a.keys + ob);
-        kd[0] = make_uint4(kv[0], kv[1], kv[2], kv[3]);
-        kd[1] = make_uint4(kv[4], kv[5], kv[6], kv[7]);
-        if (vals) {
-            uint4 *vd = (uint4 *)(a.vals + ob);
-            vd[0] = make_uint4(vv[0], vv[1], vv[2], vv[3]);
-            vd[1] = make_uint4(vv[4], vv[5], vv[6], vv[7]);
-        }
-        if (a.slot_f) *(uint2 *)(a.slot_f + ob) = make_uint2(0u, 0u);  // output o is the record's slot o
-    } else {
-#pragma unroll
-        for (int i = 0; i < EMIT_ITEMS; i++) {
-            if (ob + i >= o1) break;
-            a.keys[ob + i] = kv[i];
-            if (vals) a.vals[ob + i] = (int32_t)vv[i];
-            if (a.slot_f) a.slot_f[ob + i] = 0;
-        }
-    }
-}
-
-// tile_start[t] = first sorted intersection with tile >= t, for t in [0, T]
-__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t *keys, const uint32_t *n_ptr,
-                                                         const uint32_t *ntiles_ptr, int ntiles_host,
-                                                         int32_t *tile_start, int shift) {
-    // each thread takes 4 consecutive boundaries k0..k0+3 (one 16-byte load inside the list)
-    const uint32_t n = *n_ptr;
-    const int ntiles = ntiles_ptr ? (int)*ntiles_ptr : ntiles_host;
-    const uint32_t k0 = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (k0 > n) return;
-    uint32_t v[4];
-    if (k0 + 4 <= n) {
-        const uint4 q = *(const uint4 *)(keys + k0);
-        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = k0 + j < n ? keys[k0 + j] : 0u;
-    }
-    int tp = k0 > 0 ? (int)(keys[k0 - 1] >> shift) : -1;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t k = k0 + j;
-        if (k > n) break;
-        const int t = k < n ? (int)(v[j] >> shift) : ntiles;
-        for (int u = tp + 1; u <= t; u++) tile_start[u] = (int32_t)k;
-        tp = t;
-    }
-}
-
 // View id of each depth-sorted record, the key of one more stable pass that makes the
 // record order view-major (each view's records in depth order)
 __global__ __launch_bounds__(256) void view_keys_kernel(const int32_t *recs, const uint32_t *n_ptr, int n,
                                                        uint32_t *keys) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < *n_ptr) keys[i] = (uint32_t)(recs[i] / n);
-}
-
-// Ranges of a batch sorted by local tile, with each tile's entries grouped by view:
-// pair (t, v) owns [range_start[t V + v], range_start[t V + v + 1]), V = num_views.
-__global__ __launch_bounds__(256) void tile_ranges_views_kernel(const uint32_t *keys, const int32_t *recs,
-                                                               const uint32_t *n_ptr, int n, const BatchTable *tab,
-                                                               int32_t *range_start) {
-    const uint32_t m = *n_ptr;
-    const uint32_t V = (uint32_t)tab->num_views;
-    const int total = (int)(tab->max_view_tiles * V);
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    if (k > m) return;
-    const int c = k < m ? (int)(keys[k] * V + (uint32_t)(recs[k] / n)) : total;
-    const int cp = k > 0 ? (int)(keys[k - 1] * V + (uint32_t)(recs[k - 1] / n)) : -1;
-    for (int u = cp + 1; u <= c; u++) range_start[u] = (int32_t)k;
-}
-
-__global__ __launch_bounds__(256) void unpack_keys_kernel(const uint32_t *packed, uint32_t n, int shift,
-                                                         uint32_t *tiles, int32_t *gid) {
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const uint32_t v = packed[k];
-    tiles[k] = v >> shift;
-    gid[k] = (int32_t)(v & ((1u << shift) - 1u));
-}
-
-// The 64-bit (tile << 32 | depth bits) view of the sorted intersections
-__global__ __launch_bounds__(256) void keys64_kernel(const uint32_t *tiles, const int32_t *gid, const float *depths,
-                                                    uint32_t n, uint64_t *out) {
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-    if (k < n) out[k] = ((uint64_t)tiles[k] << 32) | (uint64_t)__float_as_uint(depths[gid[k]]);
 }
 
 // ── batched views ────────────────────────────────────────────────────────────
@@ -802,8 +618,8 @@ __global__ __launch_bounds__(256) void project_batch_kernel(BatchProjectArgs a) 
 size_t scan_partial_words(uint32_t L) { return (size_t)(L + SCAN_CHUNK - 1) / SCAN_CHUNK + 1; }
 
 void launch_scan_u32(uint32_t *a, uint32_t L, uint32_t *partial, const ScanOut &o, hipStream_t s) {
-    if (L <= 2 * SCAN_CHUNK) {  // one launch
-        scan_small_kernel<<<1, 256, 0, s>>>(a, L, o);
+    if (L <= 3 * SCAN_SMALL_CHUNK) {  // one launch
+        scan_small_kernel<<<1, SCAN_SMALL_THREADS, 0, s>>>(a, L, o);
         return;
     }
     const int nchunks = (int)((L + SCAN_CHUNK - 1) / SCAN_CHUNK);
@@ -814,8 +630,8 @@ void launch_scan_u32(uint32_t *a, uint32_t L, uint32_t *partial, const ScanOut &
 
 void launch_scan_u32_pair(uint32_t *a0, const ScanOut &o0, uint32_t *a1, const ScanOut &o1, uint32_t L,
                           uint32_t *partial0, uint32_t *partial1, hipStream_t s) {
-    if (L <= 2 * SCAN_CHUNK) {
-        scan_small_pair_kernel<<<2, 256, 0, s>>>(a0, o0, a1, o1, L);
+    if (L <= 3 * SCAN_SMALL_CHUNK) {
+        scan_small_pair_kernel<<<2, SCAN_SMALL_THREADS, 0, s>>>(a0, o0, a1, o1, L);
         return;
     }
     launch_scan_u32(a0, L, partial0, o0, s);
@@ -850,6 +666,11 @@ void launch_scan_blocks(uint32_t *sums, int nblocks, uint64_t *total, uint32_t *
     scan_blocks_kernel<<<1, 256, 0, s>>>(sums, nblocks, total, total32, zero_also);
 }
 
+void launch_slot_prepare(const SlotPrepareArgs &a, hipStream_t s) {
+    const size_t blocks = std::max((a.nwords + 255) / 256, ((size_t)a.nrec + 255) / 256);
+    if (blocks) slot_prepare_kernel<<<(unsigned)std::min<size_t>(blocks, SLOT_PREPARE_GRID), 256, 0, s>>>(a);
+}
+
 void launch_compact(const CompactArgs &a, hipStream_t s) {
     if (a.nbx > 0 && a.num_views > 0) compact_kernel<<<dim3(a.nbx, a.num_views), 256, 0, s>>>(a);
 }
@@ -865,7 +686,7 @@ size_t radix_hist_words(uint32_t n_max) {
 
 // Grid caps of the capacity-sized launches: the workgroups loop over what the device
 // count needs.
-constexpr uint32_t HIST_GRID = 2048, SCATTER_GRID = 1024, LIST_GRID = 2048;
+constexpr uint32_t HIST_GRID = 2048, SCATTER_GRID = 1024;
 
 template <typename K, int ITEMS>
 static void radix_pass_items(const K *kin, const int32_t *vin, K *kout, int32_t *vout, const uint32_t *n_dev,
@@ -897,52 +718,9 @@ void launch_radix_pass(const uint32_t *kin, const int32_t *vin, uint32_t *kout, 
     radix_pass<uint32_t>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s);
 }
 
-void launch_order_sums(const int32_t *list, const uint32_t *nvis_dev, uint32_t nvis_max, const uint32_t *count,
-                       uint32_t *sums, uint32_t *lcount, hipStream_t s) {
-    const uint32_t nb = (nvis_max + 255) / 256;
-    if (nb > 0) order_sums_kernel<<<std::min(nb, LIST_GRID), 256, 0, s>>>(list, nvis_dev, count, sums, nb, lcount);
-}
-
-void launch_keygen_offsets(const KeygenArgs &a, hipStream_t s) {
-    const uint32_t nb = (a.nvis_max + 255) / 256;
-    if (nb > 0) keygen_offsets_kernel<<<std::min(nb, LIST_GRID), 256, 0, s>>>(a);
-}
-
-void launch_keygen_emit(const KeygenArgs &a, bool batch, hipStream_t s) {
-    const uint32_t ne = (a.m_max + EMIT_CHUNK - 1) / EMIT_CHUNK;
-    if (a.nvis_max == 0 || ne == 0) return;
-    if (batch) keygen_emit_kernel<true><<<ne, 256, 0, s>>>(a);
-    else keygen_emit_kernel<false><<<ne, 256, 0, s>>>(a);
-}
-
-void launch_keygen(const KeygenArgs &a, bool batch, hipStream_t s) {
-    launch_keygen_offsets(a, s);
-    launch_keygen_emit(a, batch, s);
-}
-
-void launch_tile_ranges(const uint32_t *keys, const uint32_t *n_dev, uint32_t n_max, const uint32_t *ntiles_dev,
-                        int ntiles, int32_t *tile_start, hipStream_t s, int shift) {
-    const uint32_t nb = (n_max + 1 + 1023) / 1024;  // 4 boundaries per thread
-    tile_ranges_kernel<<<nb, 256, 0, s>>>(keys, n_dev, ntiles_dev, ntiles, tile_start, shift);
-}
-
-void launch_unpack_keys(const uint32_t *packed, uint32_t n, int shift, uint32_t *tiles, int32_t *gid, hipStream_t s) {
-    if (n) unpack_keys_kernel<<<(n + 255) / 256, 256, 0, s>>>(packed, n, shift, tiles, gid);
-}
-
-void launch_keys64(const uint32_t *tiles, const int32_t *gid, const float *depths, uint32_t n, uint64_t *out,
-                   hipStream_t s) {
-    if (n) keys64_kernel<<<(n + 255) / 256, 256, 0, s>>>(tiles, gid, depths, n, out);
-}
-
 void launch_view_keys(const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n, uint32_t *keys,
                       hipStream_t s) {
     if (n_max) view_keys_kernel<<<(n_max + 255) / 256, 256, 0, s>>>(recs, n_dev, n, keys);
-}
-
-void launch_tile_ranges_views(const uint32_t *keys, const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n,
-                              const BatchTable *tab, int32_t *range_start, hipStream_t s) {
-    tile_ranges_views_kernel<<<(n_max + 1 + 255) / 256, 256, 0, s>>>(keys, recs, n_dev, n, tab, range_start);
 }
 
 void launch_batch_project(const BatchProjectArgs &a, hipStream_t s) {

@@ -78,9 +78,7 @@ struct StepFrame {
     int n;
     uint32_t width, height;
     int tiles_x, tiles_y, ntiles;
-    uint32_t *keys_sorted;
     int32_t *gid_sorted;
-    int sort_gid_bits;
     int32_t *vis_sorted;
     int chunks;
     float bg[3];
@@ -109,9 +107,10 @@ struct msplat_hip_ctx {
     Buf splat_a, splat_b, splat_blue, depths, aabb, rect, radii, count, offsets, block_sums;
     Buf v_xy, v_conic, v_rgb, v_opac, sh_scratch, big;
     // per intersection
-    Buf keys0, keys1, vals0, vals1, slot_a, slot_b, slot_c, slot_f, hist, digit_total, keys64;
-    // visible gaussians sorted by depth, per-block counts and scan partials
-    Buf block_vis, dk0, dk1, dv0, dv1, ord_sums, scan_part, loff;
+    Buf coarse, gids, slot_a, slot_b, slot_c, slot_f, keys64;
+    Buf keys1, vals1;  // msplat_hip_radix_sort's second key and payload buffers
+    // visible gaussians sorted by depth, per-block counts, radix and scan partials, tile list scratch
+    Buf block_vis, dk0, dk1, dv0, dv1, hist, digit_total, scan_part, lrect, lists;
     // per tile / pixel
     Buf tile_start, image, final_T, final_idx, v_image, row_loss, loss_scratch;
     Buf grad_scratch;  // stands in for NULL gradient outputs of render_backward
@@ -217,14 +216,12 @@ struct msplat_hip_ctx {
     int tiles_x = 0, tiles_y = 0;
     int64_t M = 0;
     int64_t V = 0;  // visible gaussians of the frame (tile count > 0)
-    bool slot_f_clean = false;  // slot_f[0, M) is all zero: set by the key emission, cleared by a raster backward
+    bool big_listed = false;  // the frame's list of records with many intersections is built
     // How far the one-view frame in the workspace is built: the stage entry points refuse
     // to run on a frame whose inputs are missing (they would read unset device pointers).
     enum { FRAME_NONE = 0, FRAME_PROJECTED = 1, FRAME_BINNED = 2, FRAME_RASTERED = 3 };
     int frame_stage = FRAME_NONE;
-    uint32_t *keys_sorted = nullptr;  // sorted keys: tile ids, or (tile << sort_gid_bits) | id
-    int32_t *gid_sorted = nullptr;    // sorted gaussian ids (null when packed into the keys)
-    int sort_gid_bits = 0;            // > 0: the ids are the keys' low sort_gid_bits bits
+    int32_t *gid_sorted = nullptr;  // the tiles' lists of gaussian ids, in depth order
     float bg[3] = {0, 0, 0};
 
     int grow(Buf &b, size_t bytes) {
@@ -253,8 +250,8 @@ struct msplat_hip_ctx {
     ~msplat_hip_ctx() {
         if (stream) (void)hipStreamSynchronize(stream);
         Buf *all[] = {&splat_a, &splat_b, &splat_blue, &depths, &aabb, &rect, &radii, &count, &offsets, &block_sums,
-                      &v_xy, &v_conic, &v_rgb, &v_opac, &sh_scratch, &big, &keys0, &keys1, &vals0, &vals1, &slot_a, &slot_b, &slot_c, &slot_f,
-                      &hist, &digit_total, &keys64, &block_vis, &dk0, &dk1, &dv0, &dv1, &ord_sums, &scan_part, &loff, &tile_start, &image, &final_T, &final_idx, &v_image,
+                      &v_xy, &v_conic, &v_rgb, &v_opac, &sh_scratch, &big, &coarse, &gids, &keys1, &vals1, &slot_a, &slot_b, &slot_c, &slot_f,
+                      &hist, &digit_total, &keys64, &block_vis, &dk0, &dk1, &dv0, &dv1, &scan_part, &lrect, &lists, &tile_start, &image, &final_T, &final_idx, &v_image,
                       &row_loss, &loss_scratch, &scalars, &grad_scratch, &aux, &chunk_prod, &chunk_state,
                       &chunk_last, &bg_img, &out_depth, &v_aux, &adj, &v_adj, &prior_rows, &expo_part, &slot_d,
                       &big_d, &sky_acc};

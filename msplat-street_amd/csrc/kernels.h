@@ -18,7 +18,7 @@ struct Tuning {
     int fwd_batch = 256;  // forward LDS batch depth: 64, 128, 256
     int bwd_batch = 64;   // backward LDS batch depth: 32, 64, 128
     int cull = 1;         // skip a tile's gaussians whose alpha >= 1/255 ellipse misses it
-    int pack_keys = 1;    // one-view tile sort on (tile | id) keys when they fit in 32 bits
+    int pack_keys = 1;    // accepted, without effect: the tile lists are built without sort keys
 };
 
 // Per-step values of a captured one-view train step, in device memory: uploaded before
@@ -60,45 +60,65 @@ struct ScanOut {
     uint64_t *running;    // null, or the total is added here (a running count over frames)
 };
 
-// Visible records (count > 0) in id order with their depth bits as sort keys
+// Visible records (count > 0) in id order with their depth bits as sort keys, and every
+// visible record's intersection offset: the exclusive prefix of the counts in record order
 struct CompactArgs {
     int n, num_views, nbx;  // records r = v * n + g, nbx blocks of 256 per view
     const uint32_t *count;
     const float *depths;
-    const uint32_t *block_vis;  // scanned visible counts per (view, block)
+    const uint32_t *block_vis;   // scanned visible counts per (view, block)
+    const uint32_t *block_sums;  // scanned intersection counts per (view, block)
     uint32_t *dkeys;
     int32_t *dvals;
+    uint32_t *offsets;
 };
 
-// Key emission over the visible records in depth order
-struct KeygenArgs {
-    const int32_t *list;       // visible records, depth order
-    const uint32_t *nvis_ptr;  // device length of the list
-    uint32_t nvis_max;         // grid bound
+// Before a raster backward: the slots' zero flags cleared and the list of the records with
+// more than BIG_SLOTS intersections
+struct SlotPrepareArgs {
+    uint32_t *flag_words;
+    size_t nwords;
     const uint32_t *count;
-    const uint2 *rect;
-    const uint32_t *block_bases;  // scanned count sums per 256 list entries, or
-    const uint32_t *chunk_sums;   // (when not null) the sums themselves, unscanned
-    uint32_t *offsets;
-    uint32_t *loff;         // offsets in list order (nvis_max entries)
-    const uint32_t *m_ptr;  // device intersection count
-    uint32_t m_max;         // grid bound of the emission
-    uint32_t *keys;  // global tile id, or (tile id << gid_bits) | record id
-    int32_t *vals;   // record id (unused when gid_bits > 0)
-    uint32_t gid_bits;  // one view: > 0 packs the record id into the key's low bits
-    uint32_t *big_list, *big_count;  // records with count > BIG_SLOTS
-    uint8_t *slot_f;                 // null, or the slots' zero flags, cleared by the emission
-    const uint32_t *overflow;        // null, or skip everything when set
-    int tiles_x;                     // one view
-    const BatchTable *tab;           // batch: record r is in view r / n
-    int n;
+    uint32_t nrec;             // 0: the frame's list stands
+    const uint32_t *overflow;  // null, or: when set the frame is over capacity and the list stays empty
+    uint32_t *big_list, *big_count;  // big_count: 0 at the launch that builds the list
 };
+void launch_slot_prepare(const SlotPrepareArgs &a, hipStream_t s);
+
+// The per-tile lists of the visible records in depth order (tile_lists.hip)
+struct TileListArgs {
+    const int32_t *list;       // visible records, depth order (a batch: view after view)
+    const uint32_t *nvis;      // device length of the list
+    const uint32_t *overflow;  // null, or: when set the lists are empty
+    const uint2 *rect;         // per record
+    uint2 *lrect;              // scratch, one per list entry
+    uint2 *coarse;             // scratch: the supertiles' lists, at most one entry per intersection
+    int32_t *gids;             // out: the tiles' lists
+    int32_t *tile_start;       // out: list t is gids[tile_start[t], tile_start[t + 1])
+    bool direct;               // the view is one supertile
+    int tiles_x, tiles_y, nodes;  // one view; nodes = tile_list_nodes
+    const BatchTable *tab;        // batch: record r is in view r / n; global tile ids
+    const uint32_t *block_vis;    // batch: scanned visible counts, nbx per view
+    int nbx;
+    // carved from one scratch buffer (tile_list_carve)
+    uint32_t *cnt1, *wave1, *cnt2, *wave2, *unit1, *super_total, *super_start, *unit2, *plan;
+};
+uint32_t tile_list_nodes(int tiles_x, int tiles_y);  // level-1 nodes of a view
+bool tile_list_direct(int tiles_x, int tiles_y);
+size_t tile_list_scratch_words(uint32_t nodes);
+void tile_list_carve(uint32_t *scratch, uint32_t nodes, TileListArgs &a);
+// begin: what needs only the depth-ordered list; end: the rest, once the buffers hold
+// m_max intersections (ntiles: tiles of the frame, partial: scan_partial_words(ntiles + 1))
+void launch_tile_lists_begin(const TileListArgs &a, bool batch, uint32_t nodes, uint32_t nvis_max, hipStream_t s);
+void launch_tile_lists_end(const TileListArgs &a, bool batch, uint32_t nodes, uint32_t nvis_max, uint32_t m_max,
+                           uint32_t ntiles, uint32_t *partial, hipStream_t s);
+void launch_list_keys64(const int32_t *tile_start, int ntiles, const int32_t *gid, const float *depths, uint64_t *out,
+                        hipStream_t s);
 
 struct RasterArgs {
     uint32_t width, height;
     int tiles_x, tiles_y;
     const int32_t *tile_start, *gid;
-    uint32_t gid_mask;  // record id = gid[k] & gid_mask (the sort key may hold the tile id above it)
     const float4 *splat_a, *splat_b;
     const float *splat_blue;
     float bg[3];
@@ -270,9 +290,8 @@ void launch_finalize_depth(const float *depth_num, const float *final_T, uint32_
 
 // ── batched views ───────────────────────────────────────────────────────────
 // Several views of one scene go through one projection, one depth sort of the visible
-// records (then stably by view), one sort of the intersections by local tile id (each
-// tile's range then holds the views in order, each in depth order: range index
-// tile * num_views + view), one persistent rasterizer over (view, tile) items, one loss
+// records (then stably by view), one expansion into the lists of all views' tiles (global
+// tile ids, view after view), one persistent rasterizer over (view, tile) items, one loss
 // launch and one per-gaussian backward that sums over the views. Everything that
 // changes from step to step (poses, resolutions, targets, Adam scalars) is read from a
 // BatchTable in device memory, so a captured graph replays with new contents.
@@ -295,9 +314,9 @@ struct BatchTable {
     float step[6], bc2[6];
     float beta1, beta2, eps;
     uint32_t rest_active;  // SH rest coefficients per gaussian in the bands in use (max over the views)
-    uint32_t max_view_tiles;  // tiles of the largest view: ranges run over max_view_tiles * num_views
     // prefix offsets over the views (num_views + 1 entries each)
     uint32_t tile_base[MAX_VIEWS + 1], row_base[MAX_VIEWS + 1], loss_base[MAX_VIEWS + 1];
+    uint32_t node_base[MAX_VIEWS + 1];  // level-1 nodes of the tile lists
     BatchView views[MAX_VIEWS];
 };
 
@@ -310,7 +329,6 @@ struct BatchScalars {
     uint32_t big_count;  // records with more than BIG_SLOTS intersections
     uint32_t nvis;       // visible records
     uint32_t queue[2][8];  // persistent rasterizer queue heads (forward, backward) per XCD chunk
-    uint32_t total32_b, overflow_b;  // the same totals from the depth-order scan
     double loss_sum[MAX_VIEWS];
     float loss_mean[MAX_VIEWS];
 };
@@ -405,12 +423,6 @@ void launch_scan_u32(uint32_t *a, uint32_t L, uint32_t *partial, const ScanOut &
 void launch_scan_u32_pair(uint32_t *a0, const ScanOut &o0, uint32_t *a1, const ScanOut &o1, uint32_t L,
                           uint32_t *partial0, uint32_t *partial1, hipStream_t s);
 void launch_compact(const CompactArgs &a, hipStream_t s);
-// also writes each record's count in list order to lcount (the offsets kernel's loff)
-void launch_order_sums(const int32_t *list, const uint32_t *nvis_dev, uint32_t nvis_max, const uint32_t *count,
-                       uint32_t *sums, uint32_t *lcount, hipStream_t s);
-void launch_keygen_offsets(const KeygenArgs &a, hipStream_t s);  // offsets, loff, big list
-void launch_keygen_emit(const KeygenArgs &a, bool batch, hipStream_t s);  // the keys
-void launch_keygen(const KeygenArgs &a, bool batch, hipStream_t s);
 // One stable pass over the digit (key >> shift) & mask (mask at most 0xFF)
 void launch_radix_pass(const uint64_t *kin, const int32_t *vin, uint64_t *kout, int32_t *vout, const uint32_t *n_dev,
                        uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s,
@@ -419,18 +431,9 @@ void launch_radix_pass(const uint32_t *kin, const int32_t *vin, uint32_t *kout, 
                        uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s,
                        uint32_t mask = 0xFF);
 size_t radix_hist_words(uint32_t n_max);
-void launch_tile_ranges(const uint32_t *keys, const uint32_t *n_dev, uint32_t n_max, const uint32_t *ntiles_dev,
-                        int ntiles, int32_t *tile_start, hipStream_t s, int shift = 0);
-// tile ids (key >> shift) and record ids (key & (2^shift - 1)) of packed sorted keys
-void launch_unpack_keys(const uint32_t *packed, uint32_t n, int shift, uint32_t *tiles, int32_t *gid, hipStream_t s);
-void launch_keys64(const uint32_t *tiles, const int32_t *gid, const float *depths, uint32_t n, uint64_t *out,
-                   hipStream_t s);
 // batch: view ids of the depth-sorted records (record / n) as sort keys
 void launch_view_keys(const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n, uint32_t *keys,
                       hipStream_t s);
-// batch: ranges over (local tile, view) pairs, index tile * num_views + view
-void launch_tile_ranges_views(const uint32_t *keys, const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n,
-                              const BatchTable *tab, int32_t *range_start, hipStream_t s);
 int auto_chunks(int nt, int64_t m);
 void launch_raster_forward(const RasterArgs &a, const Tuning &t, hipStream_t s);
 void launch_raster_backward(const RasterArgs &a, const Tuning &t, hipStream_t s);

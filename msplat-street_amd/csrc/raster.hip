@@ -8,7 +8,7 @@ namespace msplat {
 namespace {
 
 __device__ inline TileData tile_data(const RasterArgs &a) {
-    return TileData{a.tile_start, a.gid,    a.gid_mask, a.splat_a, a.splat_b, a.splat_blue,     a.rect,
+    return TileData{a.tile_start, a.gid,    a.splat_a, a.splat_b, a.splat_blue,     a.rect,
                     a.offsets,    a.slot_a, a.slot_b,   a.slot_c,  a.slot_f,  a.slots_written, a.cull != 0,
                     a.depths,     a.slot_d};
 }
@@ -19,7 +19,7 @@ __device__ inline TileView tile_view(const RasterArgs &a) {
 }
 
 __device__ inline TileData tile_data(const BatchRasterArgs &a) {
-    return TileData{a.tile_start, a.gid,    0xFFFFFFFFu, a.splat_a, a.splat_b, a.splat_blue, a.rect,
+    return TileData{a.tile_start, a.gid,    a.splat_a, a.splat_b, a.splat_blue, a.rect,
                     a.offsets,    a.slot_a, a.slot_b,    a.slot_c,  a.slot_f,  nullptr,      a.cull != 0};
 }
 
@@ -204,8 +204,8 @@ __global__ __launch_bounds__(256 / PPT) void raster_backward_chunk_kernel(Raster
 }
 
 // Persistent forward over every (view, tile) of a batch; item t is tile t - tile_base[v]
-// of view v, whose range is number (tile * num_views + v). Every workgroup loops until
-// the queue is drained, so the grid drains on its own.
+// of view v, and list t is its list. Every workgroup loops until the queue is drained, so
+// the grid drains on its own.
 template <int FB>
 __global__ __launch_bounds__(256, 8) void raster_forward_batch_kernel(BatchRasterArgs a) {
     __shared__ uint32_t tb[MAX_VIEWS + 1];
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256, 8) void raster_forward_batch_kernel(BatchRaste
         if (t >= total) break;
         const int v = view_of(tb, nv, t);
         const int lt = (int)(t - tb[v]);
-        forward_tile<FB>(tile_view(a, v), d, lt * nv + v, lt);
+        forward_tile<FB>(tile_view(a, v), d, (int)t, lt);
     }
 }
 
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256 / PPT) void raster_backward_batch_kernel(BatchR
         if (t >= total) break;
         const int v = view_of(tb, nv, t);
         const int lt = (int)(t - tb[v]);
-        backward_tile<PPT, BB>(tile_view(a, v), d, lt * nv + v, lt);
+        backward_tile<PPT, BB>(tile_view(a, v), d, (int)t, lt);
     }
 }
 

@@ -39,7 +39,6 @@ struct TileView {
 // per-record splats and tile rectangles (in the record's view), and gradient slots.
 struct TileData {
     const int32_t *tile_start, *gid;
-    uint32_t gid_mask;  // record id = gid[k] & gid_mask
     const float4 *splat_a, *splat_b;
     const float *splat_blue;
     const uint2 *rect;
@@ -150,7 +149,7 @@ __device__ inline void forward_tile(const TileView &v, const TileData &d, int gt
         float4 A0, B0;
         float C0 = 0.f, Z0 = 0.f;
         if (threadIdx.x < FB && k < e) {
-            const int g = (int)((uint32_t)d.gid[k] & d.gid_mask);
+            const int g = d.gid[k];
             A0 = d.splat_a[g];
             B0 = d.splat_b[g];
             C0 = d.splat_blue[g];
@@ -270,7 +269,7 @@ __device__ inline int stage_forward_batch(const TileData &d, int base, int e, fl
     float4 A0, B0;
     float C0 = 0.f;
     if (threadIdx.x < FB && k < e) {
-        const int g = (int)((uint32_t)d.gid[k] & d.gid_mask);
+        const int g = d.gid[k];
         A0 = d.splat_a[g];
         B0 = d.splat_b[g];
         C0 = d.splat_blue[g];
@@ -379,8 +378,7 @@ __device__ inline void forward_chunk(const TileView &v, const TileData &d, const
 // (wave_sums9) and lanes 0..8 write the wave's totals to LDS, to be added over the waves
 // in fixed order when the batch's slots are written. One partial per wave keeps the LDS
 // footprint small enough for several waves per SIMD.
-// Every slot flag is zero when the kernel starts (the key emission clears them, or a
-// fill before a second backward of the same frame). A slot whose nine values are all
+// Every slot flag is zero when the kernel starts (slot_prepare_kernel). A slot whose nine values are all
 // zero (a record culled from the tile, behind every pixel's last contributor, or valid
 // in no pixel) is not touched: its floats stay as they are, and the slot sums skip it.
 // Skipping a zero term changes no sum: the sums start at +0, and adding +0 or -0 to +0
@@ -479,7 +477,7 @@ __device__ inline void backward_tile(const TileView &v, const TileData &d, int g
             uint32_t p = 0;
             float Z0 = 0.f;
             if (i < n) {
-                const int g = (int)((uint32_t)d.gid[start + i] & d.gid_mask);
+                const int g = d.gid[start + i];
                 A0 = d.splat_a[g];
                 B0 = d.splat_b[g];
                 C0 = d.splat_blue[g];

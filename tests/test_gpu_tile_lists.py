@@ -1,0 +1,95 @@
+"""The tiles' lists (tile_lists.hip) against a host restatement from the frame's own
+projection outputs: every tile's gaussians ascending by (depth bits, id), at the edges of
+the two expansion levels (8 tiles, 64 tiles), of the 64-entry groups, and with splats from
+under a tile to the whole view. Whole numbers: exact."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BG = np.array([0.613, 0.0101, 0.3984], np.float32)
+
+
+def _expected(ctx, f, n, tiles_x, tiles_y):
+    xy = ctx.download(f.splat_a, (n, 4), np.float32)[:, :2]
+    ext = ctx.download(f.aabb, (n, 2), np.float32)
+    rad = ctx.download(f.radii, (n,), np.int32)
+    dep = ctx.download(f.depths, (n,), np.float32)
+    t, F = np.array([tiles_x, tiles_y]), np.float32
+    vis = rad > 0
+    c, r = xy[vis] / F(16), ext[vis] / F(16)
+    lo = np.clip((c - r).astype(np.int64), 0, t)  # truncated, as a float to int conversion
+    hi = np.clip((c + r + F(1)).astype(np.int64), 0, t)
+    ids = np.nonzero(vis)[0]
+    order = np.lexsort((ids, dep[vis].view(np.uint32)))
+    lists = [[] for _ in range(tiles_x * tiles_y)]
+    for k in order:
+        for y in range(lo[k, 1], hi[k, 1]):
+            for x in range(lo[k, 0], hi[k, 0]):
+                lists[y * tiles_x + x].append(ids[k])
+    start = np.concatenate([[0], np.cumsum([len(v) for v in lists])])
+    return start, np.array([g for v in lists for g in v], np.int64)
+
+
+@pytest.mark.parametrize("W,H,n,scale", [
+    (128, 128, 1, -2.0),      # one supertile, one record
+    (128, 128, 63, -2.0), (128, 128, 64, -2.0), (128, 128, 65, -1.0),
+    (16, 16, 300, -2.5),      # one tile
+    (129, 128, 300, -2.0),    # nine tiles: the first view that takes both levels
+    (145, 271, 700, -3.0),    # odd sizes, splats around a tile
+    (1024, 1024, 500, -2.5),  # exactly one level-1 node
+    (1025, 1040, 500, -1.5),  # four nodes, three of them one tile wide
+    (2070, 40, 400, -2.0),    # three nodes side by side
+    (640, 360, 5000, -4.0),   # several units per node
+    (200, 150, 70000, -5.0),  # more entries than one group per wave holds at level 2
+])
+def test_lists_hold_each_tiles_gaussians_in_depth_order(W, H, n, scale):
+    from msplat._abi import Context
+    from msplat.backend import DeviceGaussians, render
+    from msplat.camera import look_at, make_camera
+    from msplat.scenes import random_scene
+    ctx = Context(0)
+    sc = random_scene(n + W, n, degree=0, log_scale=(scale, 0.6))
+    if n > 64:  # equal depths: the id breaks the tie
+        sc["means"][n // 2:] = sc["means"][:n - n // 2]
+    cam = make_camera(look_at((2.2, 0.5, 2.4), (0, 0, 0)), W, H, 0.9 * max(W, H), 0.9 * max(W, H))
+    dg = DeviceGaussians(ctx, sc)
+    render(ctx, dg, cam, BG)
+    f = ctx.frame()
+    start, gids = _expected(ctx, f, n, cam["tiles_x"], cam["tiles_y"])
+    assert f.num_isects == start[-1] == len(gids)
+    np.testing.assert_array_equal(ctx.download(f.tile_start, (f.num_tiles + 1,), np.int32), start)
+    np.testing.assert_array_equal(ctx.download(f.isect_gid, (len(gids),), np.int32), gids)
+    ctx.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_batched_lists_give_the_one_view_images(graph):
+    """Views of one to nine level-1 nodes in one batch (and one behind the camera): their
+    images equal the one-view renders bit for bit, also after a smaller batch shrank the
+    frame within buffers sized for more."""
+    from msplat._abi import TUNE_CHUNKS, Context, DeviceArray
+    from msplat.backend import (BatchViews, DeviceGaussians, adam_coeffs, render_batch_numpy, render_numpy,
+                                train_step_batch)
+    from msplat.camera import look_at, make_camera
+    from msplat.scenes import random_scene
+    ctx, one = Context(0), Context(0)
+    one.set_tuning(TUNE_CHUNKS, 1)
+    sc = random_scene(5, 3000, degree=1, log_scale=(-2.6, 0.7))
+    dg = DeviceGaussians(ctx, sc)
+    views = [(40, 30, (2.5, 0.6, 2.0)), (128, 128, (2.0, 0.0, 2.0)), (1025, 520, (2.4, 1.0, 1.5)),
+             (2064, 2050, (1.9, 0.3, 2.2)), (333, 217, (-2.5, 0.2, 2.0))]
+    cams = [make_camera(look_at(e, (0, 0, 0)), w, h, 0.8 * w, 0.8 * w, dtu=1) for w, h, e in views]
+    cams.append(make_camera(look_at((2.5, 0.0, 2.5), (5.0, 0.0, 5.0)), 96, 64, 90.0, 90.0, dtu=1))
+    for sub in (cams, cams[3:5], cams[:2], cams):
+        if graph:  # the same sizes through a captured step first
+            ctx.set_batch_graph(True)
+            tg = [DeviceArray(ctx, (c["H"], c["W"], 3)) for c in sub]
+            bv = BatchViews(sub, 1, [BG], tg)
+            for t in (1, 2):
+                train_step_batch(ctx, dg, bv, *adam_coeffs([0.0] * 6, t))
+        got = render_batch_numpy(ctx, dg, BatchViews(sub, 1, [BG]))
+        for c, img in zip(sub, got):
+            np.testing.assert_array_equal(img, render_numpy(one, dg, c, BG))
+    ctx.close()
+    one.close()
