@@ -77,10 +77,11 @@ __device__ inline uint32_t next_item(ItemQueue &q, uint32_t *slot) {
 
 }  // namespace
 
-// Forward kernels are capped at 64 VGPRs (8 waves per SIMD): the unrolled compositing
-// loop would otherwise hold more registers than the extra waves are worth.
+// Forward kernels are capped at this many waves' registers per SIMD: the unrolled
+// compositing loop would otherwise hold more registers than the extra waves are worth.
+constexpr int FWD_WAVES = 6;
 template <int FB, bool AUX = false>
-__global__ __launch_bounds__(256, 8) void raster_forward_kernel(RasterArgs a) {
+__global__ __launch_bounds__(FNT, FWD_WAVES) void raster_forward_kernel(RasterArgs a) {
     const int t = xcd_item(blockIdx.x, gridDim.x);
     forward_tile<FB, AUX>(tile_view(a), tile_data(a), t, t);
 }
@@ -98,7 +99,7 @@ __device__ inline ChunkView chunk_view(const RasterArgs &a, int k) {
 // Depth-chunked kernels: workgroup b runs chunk b / tiles of tile b % tiles (tiles in
 // XCD-chunked order within a chunk).
 template <int FB, bool PRODUCT>
-__global__ __launch_bounds__(256, 8) void raster_forward_chunk_kernel(RasterArgs a) {
+__global__ __launch_bounds__(FNT, FWD_WAVES) void raster_forward_chunk_kernel(RasterArgs a) {
     const int nt = a.tiles_x * a.tiles_y;
     const int k = blockIdx.x / nt, t = xcd_item(blockIdx.x % nt, nt);
     const ChunkView ch = chunk_view(a, k);
@@ -207,11 +208,11 @@ __global__ __launch_bounds__(256 / PPT) void raster_backward_chunk_kernel(Raster
 // of view v, and list t is its list. Every workgroup loops until the queue is drained, so
 // the grid drains on its own.
 template <int FB>
-__global__ __launch_bounds__(256, 8) void raster_forward_batch_kernel(BatchRasterArgs a) {
+__global__ __launch_bounds__(FNT, FWD_WAVES) void raster_forward_batch_kernel(BatchRasterArgs a) {
     __shared__ uint32_t tb[MAX_VIEWS + 1];
     __shared__ uint32_t item_slot;
     const int nv = a.num_views;
-    for (int i = threadIdx.x; i <= nv; i += 256) tb[i] = a.tab->tile_base[i];
+    for (int i = threadIdx.x; i <= nv; i += FNT) tb[i] = a.tab->tile_base[i];
     const uint32_t total = a.tab->total_tiles;
     const TileData d = tile_data(a);
     ItemQueue q{a.queue, total, 0, (int)(blockIdx.x % NUM_XCD)};
@@ -245,16 +246,16 @@ __global__ __launch_bounds__(256 / PPT) void raster_backward_batch_kernel(BatchR
 // Kernel variants by (pixels per thread, LDS batch depth), picked at launch
 template <int FB>
 static void forward_one(const RasterArgs &a, int nt, hipStream_t s) {
-    raster_forward_kernel<FB><<<nt, 256, 0, s>>>(a);
+    raster_forward_kernel<FB><<<nt, FNT, 0, s>>>(a);
 }
 
 template <int FB>
 static void forward_chunked(const RasterArgs &a, int nt, hipStream_t s) {
     const int g = nt * a.chunks;
     const dim3 pix((a.width + 15) / 16, (a.height + 15) / 16);
-    raster_forward_chunk_kernel<FB, true><<<g, 256, 0, s>>>(a);
+    raster_forward_chunk_kernel<FB, true><<<g, FNT, 0, s>>>(a);
     raster_chunk_prefix_kernel<<<pix, 256, 0, s>>>(a);
-    raster_forward_chunk_kernel<FB, false><<<g, 256, 0, s>>>(a);
+    raster_forward_chunk_kernel<FB, false><<<g, FNT, 0, s>>>(a);
     raster_chunk_merge_kernel<<<pix, 256, 0, s>>>(a);
 }
 
@@ -264,7 +265,7 @@ void launch_raster_forward(const RasterArgs &args, const Tuning &t, hipStream_t 
     const int nt = a.tiles_x * a.tiles_y;
     if (nt <= 0) return;
     if (a.aux) {  // one variant: the prior-guided path is not the tuned one
-        raster_forward_kernel<256, true><<<nt, 256, 0, s>>>(a);
+        raster_forward_kernel<256, true><<<nt, FNT, 0, s>>>(a);
         return;
     }
     if (a.chunks > 1) {
@@ -346,7 +347,7 @@ int resident_blocks(K kernel, int threads) {
 
 template <int FB>
 static int fwd_grid() {
-    static const int g = resident_blocks(raster_forward_batch_kernel<FB>, 256);
+    static const int g = resident_blocks(raster_forward_batch_kernel<FB>, FNT);
     return g;
 }
 
@@ -376,9 +377,9 @@ void launch_batch_raster_forward(const BatchRasterArgs &args, const Tuning &t, h
     a.cull = t.cull;
     zero_heads<<<1, 64, 0, s>>>(a.queue);
     const int g = batch_raster_grid(false, t);
-    if (t.fwd_batch == 64) raster_forward_batch_kernel<64><<<g, 256, 0, s>>>(a);
-    else if (t.fwd_batch == 128) raster_forward_batch_kernel<128><<<g, 256, 0, s>>>(a);
-    else raster_forward_batch_kernel<256><<<g, 256, 0, s>>>(a);
+    if (t.fwd_batch == 64) raster_forward_batch_kernel<64><<<g, FNT, 0, s>>>(a);
+    else if (t.fwd_batch == 128) raster_forward_batch_kernel<128><<<g, FNT, 0, s>>>(a);
+    else raster_forward_batch_kernel<256><<<g, FNT, 0, s>>>(a);
 }
 
 template <int PPT>
