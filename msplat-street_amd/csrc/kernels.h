@@ -233,10 +233,10 @@ void launch_metrics(const float *a, const float *b, int h, int w, float *mom, fl
                     hipStream_t s);
 
 struct KnnScratch {
-    float *bounds, *box, *sup;
-    uint64_t *codes, *codes_tmp;
+    float *bounds;
+    uint32_t *codes, *codes_tmp;
     int32_t *order, *order_tmp;
-    float4 *sorted;
+    float4 *sorted, *leaf, *mid, *top;  // points; AABBs of the tree's three levels, two float4 each
     uint32_t *hist, *digit_total, *n_dev;
 };
 size_t knn_scratch_bytes(uint32_t n);

@@ -1,20 +1,29 @@
 // Exact 3-nearest-neighbour mean distance and Gaussian initialisation
 // (msplat_knn3_mean_dist / msplat_init_gaussians, core/cpu/msplat_cpu.cpp:1499-1605).
 //
-// Points are ordered along a 30-bit Morton curve (LSD radix sort), grouped into boxes of
-// KNN_BOX consecutive points and super-boxes of KNN_SUPER boxes, each with its AABB.
-// A query seeds its three best squared distances from its Morton neighbours, then visits
-// every super-box and box whose AABB can still hold a closer point; culling uses a
-// conservative margin, so the three smallest squared distances (computed as
-// dx*dx + dy*dy + dz*dz in float, unfused) are exactly those of a brute-force search.
+// Points are ordered along a 30-bit Morton curve (LSD radix sort) and grouped into leaves of
+// 64 consecutive points, with two further levels of 64 children per node, each node with its
+// AABB. One wave searches for the 64 queries of a leaf, which lie close together: it seeds
+// every query's three best squared distances from the leaf itself, then walks the tree,
+// testing 64 children at a time (one per lane) against the leaf's own box and the largest of
+// the queries' third-best distances. Of a leaf that may hold a closer point, each query
+// tests the box itself, and the few that still need it are taken one by one, the 64 lanes
+// computing the distances to the leaf's 64 points. Culling uses a conservative margin, so
+// the three smallest squared distances (computed as dx*dx + dy*dy + dz*dz in float, unfused)
+// are exactly those of a brute-force search.
+//
+// What bounds it: the scalar steps of a wave (a leaf visited, a query taken) and the latency
+// of its dependent loads. A leaf of 64 is what one wave holds as queries and as candidates.
+// It replaced one thread per query walking boxes of 128 points, whose 64 lanes disagreed on
+// almost every box: the 475k points of a street, 2300 -> 240 us (a whole initialisation, 2450
+// -> 390 us); 20k points, 1318 -> 243 us with the ordering; 200k points in one cell of the
+// curve, beside an outlier at a thousand times their extent, 26.7 -> 3.6 ms.
 #include "common.h"
 #include "kernels.h"
 
 namespace msplat {
 
-constexpr int KNN_BOX = 128;
-constexpr int KNN_SUPER = 16;  // boxes per super-box
-constexpr int KNN_SEED = 16;   // Morton neighbours per side used to seed the search
+constexpr int KNN_FAN = 64;  // points per leaf, children per node
 
 __device__ inline uint32_t spread10(uint32_t v) {
     v &= 0x3FF;
@@ -75,7 +84,7 @@ __global__ __launch_bounds__(256) void bounds_final_kernel(const float *blk, int
     if (threadIdx.x < 6) out[threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(256) void morton_kernel(const float *pts, uint32_t n, const float *bb, uint64_t *codes,
+__global__ __launch_bounds__(256) void morton_kernel(const float *pts, uint32_t n, const float *bb, uint32_t *codes,
                                                     int32_t *idx) {
     const float lo[3] = {bb[0], bb[1], bb[2]}, hi[3] = {bb[3], bb[4], bb[5]};
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -86,7 +95,7 @@ __global__ __launch_bounds__(256) void morton_kernel(const float *pts, uint32_t 
         float t = ext > 0.f ? (pts[3 * i + a] - lo[a]) / ext : 0.f;
         q[a] = (uint32_t)fminf(fmaxf(t * 1023.f, 0.f), 1023.f);
     }
-    codes[i] = (uint64_t)(spread10(q[0]) | (spread10(q[1]) << 1) | (spread10(q[2]) << 2));
+    codes[i] = spread10(q[0]) | (spread10(q[1]) << 1) | (spread10(q[2]) << 2);
     idx[i] = (int32_t)i;
 }
 
@@ -98,89 +107,176 @@ __global__ __launch_bounds__(256) void gather_points_kernel(const float *pts, co
     sorted[i] = make_float4(pts[3 * j], pts[3 * j + 1], pts[3 * j + 2], 0.f);
 }
 
-// AABB of box b (KNN_BOX consecutive sorted points); lo in [6b..], hi in [6b+3..]
-__global__ __launch_bounds__(256) void box_bounds_kernel(const float4 *sp, uint32_t n, int nbox, float *box) {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= nbox) return;
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    const uint32_t e = min(n, (uint32_t)(b + 1) * KNN_BOX);
-    for (uint32_t i = (uint32_t)b * KNN_BOX; i < e; i++) {
-        const float4 p = sp[i];
-        lo[0] = fminf(lo[0], p.x); lo[1] = fminf(lo[1], p.y); lo[2] = fminf(lo[2], p.z);
-        hi[0] = fmaxf(hi[0], p.x); hi[1] = fmaxf(hi[1], p.y); hi[2] = fmaxf(hi[2], p.z);
-    }
-    for (int a = 0; a < 3; a++) {
-        box[6 * b + a] = lo[a];
-        box[6 * b + 3 + a] = hi[a];
-    }
+// An AABB as two float4: lo at [2 i], hi at [2 i + 1]
+struct KnnBox {
+    float lo[3], hi[3];
+};
+__device__ inline KnnBox load_box(const float4 *boxes, uint32_t i) {
+    const float4 l = boxes[2 * (size_t)i], h = boxes[2 * (size_t)i + 1];
+    return KnnBox{{l.x, l.y, l.z}, {h.x, h.y, h.z}};
 }
 
-__global__ __launch_bounds__(256) void super_bounds_kernel(const float *box, int nbox, int nsup, float *sup) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= nsup) return;
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int b = s * KNN_SUPER; b < min(nbox, (s + 1) * KNN_SUPER); b++)
-        for (int a = 0; a < 3; a++) {
-            lo[a] = fminf(lo[a], box[6 * b + a]);
-            hi[a] = fmaxf(hi[a], box[6 * b + 3 + a]);
-        }
-    for (int a = 0; a < 3; a++) {
-        sup[6 * s + a] = lo[a];
-        sup[6 * s + 3 + a] = hi[a];
-    }
-}
-
-__device__ inline void insert3(float d, float &b0, float &b1, float &b2) {
-    if (d >= b2) return;
-    if (d < b1) {
-        b2 = b1;
-        if (d < b0) {
-            b1 = b0;
-            b0 = d;
+// Boxes of groups of KNN_FAN consecutive points (LEAF) or boxes, one wave each
+template <bool LEAF>
+__global__ __launch_bounds__(256) void group_bounds_kernel(const float4 *in, uint32_t n, float4 *out) {
+    const uint32_t g = blockIdx.x * 4 + (threadIdx.x >> 6), i = g * KNN_FAN + (threadIdx.x & 63);
+    if (g * KNN_FAN >= n) return;  // the whole wave
+    KnnBox b{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+    if (i < n) {
+        if (LEAF) {
+            const float4 p = in[i];
+            b = KnnBox{{p.x, p.y, p.z}, {p.x, p.y, p.z}};
         } else {
-            b1 = d;
+            b = load_box(in, i);
         }
-    } else {
-        b2 = d;
+    }
+    for (int d = 32; d >= 1; d >>= 1)
+        for (int a = 0; a < 3; a++) {
+            b.lo[a] = fminf(b.lo[a], __shfl_xor(b.lo[a], d));
+            b.hi[a] = fmaxf(b.hi[a], __shfl_xor(b.hi[a], d));
+        }
+    if ((threadIdx.x & 63) == 0) {
+        out[2 * (size_t)g] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.f);
+        out[2 * (size_t)g + 1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.f);
     }
 }
 
-// squared distance from q to an AABB, in double, shrunk by a relative margin so that a
-// float-rounded point distance can never be smaller than the culling bound
-__device__ inline bool box_may_hold(const float *bx, float qx, float qy, float qz, float best) {
-    const double dx = fmax(0.0, fmax((double)bx[0] - qx, (double)qx - bx[3]));
-    const double dy = fmax(0.0, fmax((double)bx[1] - qy, (double)qy - bx[4]));
-    const double dz = fmax(0.0, fmax((double)bx[2] - qz, (double)qz - bx[5]));
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    return d2 * (1.0 - 1e-5) <= (double)best;
+__device__ inline float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ inline KnnBox lane_box(const KnnBox &b, int l) {
+    KnnBox r;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        r.lo[a] = lane_value(b.lo[a], l);
+        r.hi[a] = lane_value(b.hi[a], l);
+    }
+    return r;
+}
+
+// Whether two boxes may hold points at a float-rounded squared distance below `best`:
+// every rounding here and in a point distance is below 1e-6 of its value, and the bound is
+// shrunk by 1e-5 (an underflow makes it smaller still).
+__device__ inline bool boxes_within(const KnnBox &p, const KnnBox &q, float best) {
+    float d2 = 0.f;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float d = fmaxf(0.f, fmaxf(p.lo[a] - q.hi[a], q.lo[a] - p.hi[a]));
+        d2 += d * d;
+    }
+    return d2 * (1.f - 1e-5f) < best;
+}
+
+// d into the sorted three smallest b0 <= b1 <= b2
+__device__ inline void insert3(float d, float &b0, float &b1, float &b2) {
+    b2 = __builtin_amdgcn_fmed3f(b1, b2, d);
+    b1 = __builtin_amdgcn_fmed3f(b0, b1, d);
+    b0 = fminf(b0, d);
+}
+
+__device__ inline float wave_max(float v) {
+    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
+    return v;
 }
 
 __global__ __launch_bounds__(256) void knn3_kernel(const float4 *sp, const int32_t *order, uint32_t n,
-                                                  const float *box, int nbox, const float *sup, int nsup,
-                                                  float *mean_dist) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float4 q = sp[i];
-    float b0 = INFINITY, b1 = INFINITY, b2 = INFINITY;
-    auto visit = [&](uint32_t j) {
-        if (j == i) return;
-        const float4 p = sp[j];
-        const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        insert3(dx * dx + dy * dy + dz * dz, b0, b1, b2);
+                                                  const float4 *leaf, uint32_t nleaf, const float4 *mid, uint32_t nmid,
+                                                  const float4 *top, uint32_t ntop, float *mean_dist) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t g = blockIdx.x * 4 + (threadIdx.x >> 6);  // the wave's leaf
+    if (g >= nleaf) return;
+    const uint32_t i = g * KNN_FAN + lane;
+    float4 q = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+    if (i < n) q = sp[i];
+    const bool live = isfinite(q.x) && isfinite(q.y) && isfinite(q.z);  // else no point is at a finite distance
+    float b0 = INFINITY, b1 = INFINITY, b2 = live ? INFINITY : -INFINITY;
+    // the leaf's own points
+    for (int k = 0; k < KNN_FAN && g * KNN_FAN + k < n; k++) {
+        const float dx = lane_value(q.x, k) - q.x, dy = lane_value(q.y, k) - q.y, dz = lane_value(q.z, k) - q.z;
+        const float d = dx * dx + dy * dy + dz * dz;
+        if (live && lane != k && d < b2) insert3(d, b0, b1, b2);
+    }
+    const KnnBox own = load_box(leaf, g);
+    float best = wave_max(b2);  // of the live queries
+    const KnnBox me{{q.x, q.y, q.z}, {q.x, q.y, q.z}};
+    // leaf c with box b (both the same in every lane)
+    auto visit = [&](uint32_t c, const KnnBox &b) {
+        uint64_t need = __ballot(live && boxes_within(b, me, b2));
+        if (need == 0) return;
+        const uint32_t j = c * KNN_FAN + lane;
+        float4 p = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        if (j < n) p = sp[j];
+        while (need) {
+            const int t = __builtin_ctzll(need);
+            need &= need - 1;
+            const float dx = p.x - lane_value(q.x, t), dy = p.y - lane_value(q.y, t), dz = p.z - lane_value(q.z, t);
+            const float d = dx * dx + dy * dy + dz * dz;
+            uint64_t closer = __ballot(d < lane_value(b2, t));
+            while (closer) {
+                const int s = __builtin_ctzll(closer);
+                closer &= closer - 1;
+                const float ds = lane_value(d, s);
+                if (lane == t) insert3(ds, b0, b1, b2);
+            }
+        }
     };
-    // seed from the Morton neighbours, then the culled exhaustive search; the seed range
-    // is skipped there so that no point is inserted twice
-    const uint32_t s0 = i > KNN_SEED ? i - KNN_SEED : 0, s1 = min(n, i + KNN_SEED + 1);
-    for (uint32_t j = s0; j < s1; j++) visit(j);
-    for (int s = 0; s < nsup; s++) {
-        if (!box_may_hold(sup + 6 * s, q.x, q.y, q.z, b2)) continue;
-        for (int b = s * KNN_SUPER; b < min(nbox, (s + 1) * KNN_SUPER); b++) {
-            if (!box_may_hold(box + 6 * b, q.x, q.y, q.z, b2)) continue;
-            const uint32_t e = min(n, (uint32_t)(b + 1) * KNN_BOX);
-            for (uint32_t j = (uint32_t)b * KNN_BOX; j < e; j++)
-                if (j < s0 || j >= s1) visit(j);
+    // neighbours along the curve first, then the own middle node: they shrink the bound
+    if (g > 0) visit(g - 1, load_box(leaf, g - 1));
+    if (g + 1 < nleaf) visit(g + 1, load_box(leaf, g + 1));
+    best = wave_max(b2);
+    const uint32_t home = g / KNN_FAN;
+    // (a leaf visited twice would insert its points twice: the neighbours are left out)
+    auto skip = [&](uint32_t c) { return c == g || c + 1 == g || c == g + 1; };
+    // Middle node m with box mb. A leaf whose points straddle a jump of the curve has a box
+    // that overlaps most of the tree (alone, it took 0.8 ms at 475k points), so the queries
+    // that need the node are found first, and its leaves are tested against those alone.
+    auto walk_mid = [&](uint32_t m, const KnnBox &mb) {
+        const bool need = live && boxes_within(mb, me, b2);
+        if (__ballot(need) == 0) return;
+        KnnBox near;
+        float far2 = need ? b2 : -INFINITY;
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            near.lo[a] = need ? me.lo[a] : INFINITY;
+            near.hi[a] = need ? me.hi[a] : -INFINITY;
+        }
+        for (int d = 32; d >= 1; d >>= 1) {
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                near.lo[a] = fminf(near.lo[a], __shfl_xor(near.lo[a], d));
+                near.hi[a] = fmaxf(near.hi[a], __shfl_xor(near.hi[a], d));
+            }
+            far2 = fmaxf(far2, __shfl_xor(far2, d));
+        }
+        const uint32_t c = m * KNN_FAN + lane;
+        KnnBox b{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+        if (c < nleaf) b = load_box(leaf, c);
+        uint64_t todo = __ballot(c < nleaf && !skip(c) && boxes_within(b, near, far2));
+        while (todo) {
+            const int t = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            visit(m * KNN_FAN + t, lane_box(b, t));
+        }
+        best = wave_max(b2);
+    };
+    walk_mid(home, load_box(mid, home));
+    for (uint32_t t0 = 0; t0 < ntop; t0 += KNN_FAN) {
+        const uint32_t t = t0 + lane;
+        uint64_t tops = __ballot(t < ntop && boxes_within(load_box(top, t < ntop ? t : 0), own, best));
+        while (tops) {
+            const uint32_t u = t0 + __builtin_ctzll(tops);
+            tops &= tops - 1;
+            const uint32_t m = u * KNN_FAN + lane;
+            const KnnBox b = load_box(mid, m < nmid ? m : 0);
+            uint64_t mids = __ballot(m < nmid && m != home && boxes_within(b, own, best));
+            while (mids) {
+                const int k = __builtin_ctzll(mids);
+                mids &= mids - 1;
+                walk_mid(u * KNN_FAN + k, lane_box(b, k));
+            }
         }
     }
+    if (i >= n) return;
     float sum = 0.f, cnt = 0.f;
     if (isfinite(b0)) { sum += sqrtf(b0); cnt += 1.f; }
     if (isfinite(b1)) { sum += sqrtf(b1); cnt += 1.f; }
@@ -219,39 +315,39 @@ int knn3_launch(const float *pts, uint32_t n, float *mean_dist, KnnScratch &w, h
     for (int shift = 0; shift < 30; shift += 8)
         launch_radix_pass(w.codes, w.order, w.codes_tmp, w.order_tmp, w.n_dev, n, shift, w.hist, w.digit_total, s),
             std::swap(w.codes, w.codes_tmp), std::swap(w.order, w.order_tmp);
-    const int nbox = (int)((n + KNN_BOX - 1) / KNN_BOX), nsup = (nbox + KNN_SUPER - 1) / KNN_SUPER;
+    const uint32_t nleaf = (n + KNN_FAN - 1) / KNN_FAN, nmid = (nleaf + KNN_FAN - 1) / KNN_FAN,
+                   ntop = (nmid + KNN_FAN - 1) / KNN_FAN;
     gather_points_kernel<<<nb, 256, 0, s>>>(pts, w.order, n, w.sorted);
-    box_bounds_kernel<<<(nbox + 255) / 256, 256, 0, s>>>(w.sorted, n, nbox, w.box);
-    super_bounds_kernel<<<(nsup + 255) / 256, 256, 0, s>>>(w.box, nbox, nsup, w.sup);
-    knn3_kernel<<<nb, 256, 0, s>>>(w.sorted, w.order, n, w.box, nbox, w.sup, nsup, mean_dist);
+    group_bounds_kernel<true><<<(nleaf + 3) / 4, 256, 0, s>>>(w.sorted, n, w.leaf);
+    group_bounds_kernel<false><<<(nmid + 3) / 4, 256, 0, s>>>(w.leaf, nleaf, w.mid);
+    group_bounds_kernel<false><<<(ntop + 3) / 4, 256, 0, s>>>(w.mid, nmid, w.top);
+    knn3_kernel<<<(nleaf + 3) / 4, 256, 0, s>>>(w.sorted, w.order, n, w.leaf, nleaf, w.mid, nmid, w.top, ntop, mean_dist);
     return 0;
 }
 
+static size_t knn_boxes(uint32_t n) {  // of all three levels
+    const size_t nleaf = ((size_t)n + KNN_FAN - 1) / KNN_FAN, nmid = (nleaf + KNN_FAN - 1) / KNN_FAN;
+    return nleaf + nmid + (nmid + KNN_FAN - 1) / KNN_FAN;
+}
+
 size_t knn_scratch_bytes(uint32_t n) {
-    const size_t nbox = (n + KNN_BOX - 1) / KNN_BOX, nsup = (nbox + KNN_SUPER - 1) / KNN_SUPER;
-    return 6 * 1025 * 4 + 2 * 8 * (size_t)n + 2 * 4 * (size_t)n + 16 * (size_t)n + 6 * 4 * (nbox + nsup) +
-           4 * radix_hist_words(n) + 4 * 256 + 64 + 16 * 8;
+    return 16 * (size_t)n + 32 * knn_boxes(n) + 4 * 4 * (size_t)n + 6 * 1025 * 4 + 4 * radix_hist_words(n) + 4 * 256 + 64;
 }
 
 void knn_scratch_carve(void *base, uint32_t n, KnnScratch &w) {
-    const size_t nbox = (n + KNN_BOX - 1) / KNN_BOX, nsup = (nbox + KNN_SUPER - 1) / KNN_SUPER;
-    char *p = (char *)base;
-    auto take = [&](size_t bytes) {
-        char *r = p;
-        p += (bytes + 15) & ~(size_t)15;
-        return (void *)r;
-    };
-    w.bounds = (float *)take(6 * 1025 * 4);
-    w.codes = (uint64_t *)take(8 * (size_t)n);
-    w.codes_tmp = (uint64_t *)take(8 * (size_t)n);
-    w.order = (int32_t *)take(4 * (size_t)n);
-    w.order_tmp = (int32_t *)take(4 * (size_t)n);
-    w.sorted = (float4 *)take(16 * (size_t)n);
-    w.box = (float *)take(6 * 4 * nbox);
-    w.sup = (float *)take(6 * 4 * nsup);
-    w.hist = (uint32_t *)take(4 * radix_hist_words(n));
-    w.digit_total = (uint32_t *)take(4 * 256);
-    w.n_dev = (uint32_t *)take(64);
+    const size_t nleaf = ((size_t)n + KNN_FAN - 1) / KNN_FAN, nmid = (nleaf + KNN_FAN - 1) / KNN_FAN;
+    w.sorted = (float4 *)base;
+    w.leaf = w.sorted + n;
+    w.mid = w.leaf + 2 * nleaf;
+    w.top = w.mid + 2 * nmid;
+    w.codes = (uint32_t *)(w.leaf + 2 * knn_boxes(n));
+    w.codes_tmp = w.codes + n;
+    w.order = (int32_t *)(w.codes_tmp + n);
+    w.order_tmp = w.order + n;
+    w.bounds = (float *)(w.order_tmp + n);
+    w.hist = (uint32_t *)(w.bounds + 6 * 1025);
+    w.digit_total = w.hist + radix_hist_words(n);
+    w.n_dev = w.digit_total + 256;
 }
 
 void launch_init_gaussians(const float *md, const uint8_t *rgb, uint32_t n, uint32_t seed, float logit, float *scales,

@@ -160,6 +160,53 @@ def test_knn_large_street_cloud(ctx, oracle):
     np.testing.assert_array_equal(out.numpy(), oracle.knn3(pts))
 
 
+def _knn_brute(pts):
+    """float32, dx*dx + dy*dy + dz*dz unfused, over the finite distances alone."""
+    out = np.ones(len(pts), np.float32)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for i, p in enumerate(pts):
+            d = pts - p
+            d2 = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+            d2[i] = np.inf
+            d2 = np.sort(d2[np.isfinite(d2)])[:3]
+            if len(d2):
+                r = np.sqrt(d2)
+                out[i] = sum(r[1:], r[0]) / np.float32(len(d2))
+    return out
+
+
+@pytest.mark.parametrize("n,kind", [(63, "uniform"), (64, "uniform"), (65, "uniform"), (129, "nonfinite"),
+                                    (4095, "uniform"), (4097, "nonfinite"), (4160, "outlier"), (6000, "repeats")])
+def test_knn_tree_edges(ctx, n, kind):
+    """Around the 64 points of a leaf and the 64 leaves of a middle node; points that are not
+    finite (no neighbour of any other, and alone themselves); an outlier that squeezes all
+    others into few cells of the curve; every point many times. Bit-exact."""
+    from msplat._abi import DeviceArray, check, lib
+    rng = np.random.default_rng(n)
+    pts = rng.uniform(-3, 3, (n, 3)).astype(np.float32)
+    if kind == "nonfinite":
+        pts[5, 1], pts[70], pts[n - 1, 2], pts[100, 0] = np.nan, np.inf, -np.inf, np.nan
+    if kind == "outlier":
+        pts[17] = 3e5
+    if kind == "repeats":
+        pts = pts[rng.integers(0, 1500, n)]
+    dp = DeviceArray.from_numpy(ctx, pts)
+    out = DeviceArray(ctx, (n,))
+    check(lib().msplat_hip_knn3_mean_dist(ctx.ptr, dp.ptr, n, out.ptr))
+    np.testing.assert_array_equal(out.numpy(), _knn_brute(pts))
+
+
+@pytest.mark.parametrize("n", [262_144, 262_209])
+def test_knn_second_top_node(ctx, oracle, n):
+    """The last size with one top node's worth of points, and one with a second."""
+    from msplat._abi import DeviceArray, check, lib
+    pts = np.random.default_rng(n).uniform(-3, 3, (n, 3)).astype(np.float32)
+    dp = DeviceArray.from_numpy(ctx, pts)
+    out = DeviceArray(ctx, (n,))
+    check(lib().msplat_hip_knn3_mean_dist(ctx.ptr, dp.ptr, n, out.ptr))
+    np.testing.assert_array_equal(out.numpy(), oracle.knn3(pts))
+
+
 def test_init_gaussians_matches_golden(ctx):
     from msplat._abi import DeviceArray, check, lib
     d = golden("knn_init")
