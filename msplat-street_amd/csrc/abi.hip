@@ -149,9 +149,12 @@ int do_bin(msplat_hip_ctx *ctx, uint32_t cap = 0) {
     ctx->big_listed = false;
     uint32_t *dki = (uint32_t *)ctx->dk0.p, *dko = (uint32_t *)ctx->dk1.p;
     int32_t *dvi = (int32_t *)ctx->dv0.p, *dvo = (int32_t *)ctx->dv1.p;
+    const bool direct = tile_list_direct(ctx->tiles_x, ctx->tiles_y);
+    const ListEntries entries{(const uint2 *)ctx->rect.p, (uint2 *)ctx->lrect.p, direct};
     for (int shift = 0; shift < 32; shift += 8) {
         launch_radix_pass(dki, dvi, dko, dvo, ctx->d_vis32(), (uint32_t)Nc, shift, (uint32_t *)ctx->hist.p,
-                          (uint32_t *)ctx->digit_total.p, s);
+                          (uint32_t *)ctx->digit_total.p, s, 0xFF,
+                          shift == 24 ? entries : ListEntries{nullptr, nullptr, false});
         std::swap(dki, dko);
         std::swap(dvi, dvo);
     }
@@ -162,10 +165,9 @@ int do_bin(msplat_hip_ctx *ctx, uint32_t cap = 0) {
     t.list = dvi;
     t.nvis = ctx->d_vis32();
     t.overflow = cap ? ctx->d_overflow() : nullptr;
-    t.rect = (const uint2 *)ctx->rect.p;
-    t.lrect = (uint2 *)ctx->lrect.p;
+    t.lrect = (const uint2 *)ctx->lrect.p;
     t.tile_start = (int32_t *)ctx->tile_start.p;
-    t.direct = tile_list_direct(ctx->tiles_x, ctx->tiles_y);
+    t.direct = direct;
     t.tiles_x = ctx->tiles_x;
     t.tiles_y = ctx->tiles_y;
     t.nodes = (int)nodes;

@@ -11,6 +11,8 @@
 // (they add exact zeros). Built with -ffp-contract=off.
 #include <cstring>
 
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 #include "proj_math.h"
@@ -26,7 +28,12 @@ __device__ inline void adam_step(float &p, float &m1, float &m2, float g, float 
     m2 = v;
 }
 
-constexpr int BIG_REDUCE_GRID = 2048;  // 8 waves per SIMD
+// Workgroups of big_reduce_kernel for records that may be big: few enough records each
+// that the device deals them out as workgroups end (the street: 43 us, 2048 workgroups 49,
+// 16384 48), and one per 32 in small frames, where most find none (a step of 20k
+// gaussians: 279 us with 5000 workgroups, 274 with 625).
+constexpr size_t BIG_REDUCE_GRID = 8192;
+static unsigned big_reduce_grid(size_t nrec) { return (unsigned)std::min((nrec + 31) / 32, BIG_REDUCE_GRID); }
 
 // The zero flags of the c <= BIG_SLOTS slots from o as a mask (bit k: slot o + k was
 // written), from the at most nine aligned words that hold them. The words also hold
@@ -234,71 +241,178 @@ __global__ __launch_bounds__(256) void backward_kernel(BackwardArgs a) {
     }
 }
 
-// Slot sums of the gaussians with more than BIG_SLOTS intersections, one wave each
-// (grid-stride over the device-side list; every wave exits when the list is done).
-// Lane l adds the written slots among l, l + 64, ... in order, in rounds of four slots
-// whose flag and value loads are in flight together; the nine lane sums (ten with depth
-// slots) are added over the wave by wave_sums9 (wave_sums10). The next record's id and slot range are loaded while this one
-// is summed.
-__global__ __launch_bounds__(256) void big_reduce_kernel(BackwardArgs a) {
-    const uint32_t nbig = *a.big_count;
-    const int lane = threadIdx.x & 63;
-    const SumLanes sl(lane);
-    const uint32_t wave = (blockIdx.x * 256 + threadIdx.x) >> 6, nwaves = (gridDim.x * 256) >> 6;
-    uint32_t g = wave < nbig ? a.big_list[wave] : 0u;
-    uint32_t o = 0, end = 0;
-    if (wave < nbig) {
-        o = a.offsets[g];
-        end = o + a.count[g];
+// A wave sums BR_SLOTS consecutive slots of a record at a time: their zero flags, from any
+// alignment, are at most 256 words, four a lane.
+constexpr int BR_ROUNDS = 4;
+constexpr uint32_t BR_SLOTS = 64 * 4 * BR_ROUNDS - 4;
+
+// Word 64 r + lane of the flags of the c slots from o, zero past the last
+__device__ inline void load_flags(const uint8_t *sf, uint32_t o, uint32_t c, int lane, uint32_t f[BR_ROUNDS]) {
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(sf) + (o >> 2);
+    const uint32_t nw = c ? ((o & 3u) + c + 3u) >> 2 : 0u;
+#pragma unroll
+    for (int r = 0; r < BR_ROUNDS; r++) f[r] = 64u * r + lane < nw ? w[64 * r + lane] : 0u;
+}
+
+// Adds the written slots among the c <= BR_SLOTS from o, whose flag words are f, to the
+// lane's sums v: they are listed in LDS in slot order, and lane l takes those of rank l,
+// l + 64, ..., whatever the alignment of o. Calls `next` once the first values' loads are
+// on their way. Returns how many there were. (The words' bytes outside the range belong to
+// other records, or were never written: slot_mask.)
+template <class Next>
+__device__ inline uint32_t sum_written(const BackwardArgs &a, uint32_t o, uint32_t c, const uint32_t f[BR_ROUNDS],
+                                       uint16_t *list, int lane, float v[10], Next next) {
+    const int lo = (int)(o & 3u), hi = lo + (int)c;
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int r = 0; r < BR_ROUNDS; r++) {
+        if (256 * r >= hi) break;
+        const int b = 4 * (64 * r + lane);  // the word's first byte
+        uint32_t nz = ((((f[r] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | f[r]) & 0x80808080u) >> 7;
+        nz = (nz | (nz >> 7) | (nz >> 14) | (nz >> 21)) & 0xFu;
+        if (b < lo) nz &= 0xFu << lo;  // b is 0 then
+        if (b + 4 > hi) nz = b < hi ? nz & ((1u << (hi - b)) - 1u) : 0u;
+        uint32_t pos = cnt;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint64_t m = __ballot((nz >> k) & 1u);
+            pos += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            cnt += (uint32_t)__popcll(m);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if ((nz >> k) & 1u) list[pos + (uint32_t)__popc(nz & ((1u << k) - 1u))] = (uint16_t)(b + k);
     }
-    for (uint32_t i = wave; i < nbig; i += nwaves) {
-        // the next record's id and slot range, loaded while this one is summed
-        const uint32_t gn = i + nwaves < nbig ? a.big_list[i + nwaves] : 0u;
-        uint32_t on = 0, cn = 0;
-        if (i + nwaves < nbig) {
-            on = a.offsets[gn];
-            cn = a.count[gn];
-        }
-        float v[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, vd = 0.f;
-        for (uint32_t p0 = o + lane; p0 < end; p0 += 256) {
-            bool f[4];
+    wave_sync();
+    const uint32_t base = o & ~3u;
+    constexpr int U = 2;
+    for (uint32_t t0 = 0; t0 < cnt; t0 += 64 * U) {
+        float4 A[U], B[U];
+        float C[U], D[U];
 #pragma unroll
-            for (int u = 0; u < 4; u++) f[u] = p0 + 64 * u < end && a.slot_f[p0 + 64 * u] != 0;
-            if (a.slot_d)
-#pragma unroll
-                for (int u = 0; u < 4; u++) vd += f[u] ? a.slot_d[p0 + 64 * u] : 0.f;
-            float4 A[4], B[4];
-            float Cs[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                if (f[u]) {
-                    A[u] = a.slot_a[p0 + 64 * u];
-                    B[u] = a.slot_b[p0 + 64 * u];
-                    Cs[u] = a.slot_c[p0 + 64 * u];
-                } else {
-                    A[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    B[u] = A[u];
-                    Cs[u] = 0.f;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                v[0] += A[u].x; v[1] += A[u].y; v[2] += A[u].z; v[3] += A[u].w;
-                v[4] += B[u].x; v[5] += B[u].y; v[6] += B[u].z; v[7] += B[u].w;
-                v[8] += Cs[u];
+        for (int u = 0; u < U; u++) {
+            const uint32_t t = t0 + 64 * u + lane;
+            A[u] = B[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            C[u] = D[u] = 0.f;
+            if (t < cnt) {
+                const uint32_t p = base + list[t];
+                A[u] = a.slot_a[p];
+                B[u] = a.slot_b[p];
+                C[u] = a.slot_c[p];
+                if (a.slot_d) D[u] = a.slot_d[p];
             }
         }
-        // with depth slots the tenth sum rides with the ninth: lane 9 ends with its total
-        const float t = a.slot_d ? wave_sums10(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], vd)
-                                 : wave_sums9(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
+        if (t0 == 0) next();
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u && t0 + 64 * u >= cnt) break;
+            v[0] += A[u].x; v[1] += A[u].y; v[2] += A[u].z; v[3] += A[u].w;
+            v[4] += B[u].x; v[5] += B[u].y; v[6] += B[u].z; v[7] += B[u].w;
+            v[8] += C[u];
+            v[9] += D[u];
+        }
+    }
+    if (cnt == 0) next();
+    wave_sync();  // the list is free again
+    return cnt;
+}
+
+// Slot sums of the gaussians with more than BIG_SLOTS intersections (about one slot in six
+// is written), one wave each, grid-stride over the device-side list; the nine lane sums
+// (ten with depth slots) are added over the wave by wave_sums9 (wave_sums10). The next
+// record's flags are loaded while this one's values are on their way, and its id and slot
+// range a record earlier. Records of more than BR_SLOTS slots, up to every tile of the view,
+// are left to the end, where the workgroup's waves sum BR_SLOTS slots of one each in turn.
+//
+// Bound by the round trips of a record (flags, then values) and by the largest records.
+// Reading all slots' flags byte by byte and the written values four strided slots at a time,
+// one wave for a record of any size, took 56 us at 55k records of 10.5M slots (the street at
+// 1264x832; now 43) and 510 us for a batch of 8 views (now 450 to 500).
+constexpr uint32_t BR_HUGE = 2;  // such records that a workgroup sets aside; its waves sum any others
+__global__ __launch_bounds__(256) void big_reduce_kernel(BackwardArgs a) {
+    __shared__ uint16_t lists[4][BR_SLOTS + 4];
+    __shared__ uint32_t huge[BR_HUGE], nhuge;
+    __shared__ float part[4][10];
+    const uint32_t nbig = *a.big_count;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint16_t *list = lists[w];
+    const SumLanes sl(lane);
+    if (threadIdx.x == 0) nhuge = 0;
+    __syncthreads();
+    auto scalar = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+    const uint32_t wave = scalar(blockIdx.x * 4 + w), nwaves = gridDim.x * 4;
+    auto id = [&](uint32_t i) { return i < nbig ? a.big_list[i] : 0xFFFFFFFFu; };
+    auto load_range = [&](uint32_t g, uint32_t &o, uint32_t &c) {
+        o = c = 0;
+        if (g != 0xFFFFFFFFu) {
+            o = a.offsets[g];
+            c = a.count[g];
+        }
+    };
+    auto sums = [&](const float v[10]) {  // with depth slots the tenth sum rides with the ninth: lane 9 ends with it
+        return a.slot_d ? wave_sums10(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9])
+                        : wave_sums9(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
+    };
+    auto store = [&](uint32_t g, float t) {
         if (a.slot_d && lane == 9) a.big_d[g] = t;
         if (lane < 9) {
             float *dst = sl.q < 4 ? &a.big_a[g].x + sl.q : sl.q < 8 ? &a.big_b[g].x + (sl.q - 4) : &a.big_c[g];
             *dst = t;
         }
-        g = gn;
-        o = on;
-        end = on + cn;
+    };
+    uint32_t g = scalar(id(wave)), gn = scalar(id(wave + nwaves)), g2 = scalar(id(wave + 2 * nwaves)), o, c, on, cn;
+    load_range(g, o, c);
+    load_range(gn, on, cn);
+    o = scalar(o); c = scalar(c); on = scalar(on); cn = scalar(cn);
+    uint32_t f[BR_ROUNDS];
+    load_flags(a.slot_f, o, min(c, BR_SLOTS), lane, f);
+    for (uint32_t i = wave; i < nbig; i += nwaves) {
+        uint32_t o2, c2;
+        load_range(g2, o2, c2);
+        const uint32_t g3 = id(i + 3 * nwaves);
+        uint32_t at = BR_HUGE;
+        if (c > BR_SLOTS) {
+            if (lane == 0) at = atomicAdd(&nhuge, 1u);
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (at < BR_HUGE && lane == 0) huge[at] = g;
+        }
+        if (at < BR_HUGE) {
+            load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
+        } else {
+            float v[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            uint32_t written = 0;
+            for (uint32_t s = 0; s < c; s += BR_SLOTS) {  // the next flags: this record's, or the next one's
+                const bool more = s + BR_SLOTS < c;
+                uint32_t fc[BR_ROUNDS];
+#pragma unroll
+                for (int r = 0; r < BR_ROUNDS; r++) fc[r] = f[r];
+                written += sum_written(a, o + s, min(c - s, BR_SLOTS), fc, list, lane, v, [&] {
+                    if (more) load_flags(a.slot_f, o + s + BR_SLOTS, min(c - s - BR_SLOTS, BR_SLOTS), lane, f);
+                    else load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
+                });
+            }
+            store(g, written ? sums(v) : 0.f);
+        }
+        g = gn; o = on; c = cn;
+        gn = g2; on = scalar(o2); cn = scalar(c2);
+        g2 = scalar(g3);
+    }
+    __syncthreads();
+    const uint32_t nh = min(nhuge, BR_HUGE);
+    for (uint32_t k = 0; k < nh; k++) {
+        const uint32_t h = scalar(huge[k]), ho = scalar(a.offsets[h]), hc = scalar(a.count[h]);
+        float v[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (uint32_t s = w * BR_SLOTS; s < hc; s += 4 * BR_SLOTS) {
+            load_flags(a.slot_f, ho + s, min(hc - s, BR_SLOTS), lane, f);
+            sum_written(a, ho + s, min(hc - s, BR_SLOTS), f, list, lane, v, [] {});
+        }
+        const float t = sums(v);
+        if (lane < 9) part[w][sl.q] = t;
+        if (lane == 9) part[w][9] = t;
+        __syncthreads();
+        if (w == 0) store(h, lane < 9 ? ((part[0][sl.q] + part[1][sl.q]) + part[2][sl.q]) + part[3][sl.q]
+                                      : ((part[0][9] + part[1][9]) + part[2][9]) + part[3][9]);
+        __syncthreads();
     }
 }
 
@@ -485,7 +599,8 @@ __global__ __launch_bounds__(256) void batch_adam_kernel(float *p, float *m1, fl
 
 void launch_big_reduce_records(const uint32_t *big_list, const uint32_t *big_count, const uint32_t *offsets,
                                const uint32_t *count, const float4 *slot_a, const float4 *slot_b, const float *slot_c,
-                               const uint8_t *slot_f, float4 *big_a, float4 *big_b, float *big_c, hipStream_t s) {
+                               const uint8_t *slot_f, float4 *big_a, float4 *big_b, float *big_c, size_t nrec, hipStream_t s) {
+    if (nrec == 0) return;
     BackwardArgs a;
     memset(&a, 0, sizeof a);
     a.big_list = big_list;
@@ -499,7 +614,7 @@ void launch_big_reduce_records(const uint32_t *big_list, const uint32_t *big_cou
     a.big_a = big_a;
     a.big_b = big_b;
     a.big_c = big_c;
-    big_reduce_kernel<<<BIG_REDUCE_GRID, 256, 0, s>>>(a);
+    big_reduce_kernel<<<big_reduce_grid(nrec), 256, 0, s>>>(a);
 }
 
 void launch_batch_backward(const BatchBackwardArgs &a, hipStream_t s) {
@@ -518,7 +633,7 @@ void launch_backward(const BackwardArgs &a, BackwardMode mode, hipStream_t s) {
     if (nb == 0) return;
     const size_t ne = (size_t)a.n * (sh_bases(a.cam.degree) - 1) * 3;
     const int nbe = (int)((ne + 255) / 256);
-    big_reduce_kernel<<<BIG_REDUCE_GRID, 256, 0, s>>>(a);
+    big_reduce_kernel<<<big_reduce_grid((size_t)a.n), 256, 0, s>>>(a);
     if (mode == BWD_ADAM) {
         if (a.sp) {
             backward_kernel<BWD_ADAM, true><<<nb, 256, 0, s>>>(a);

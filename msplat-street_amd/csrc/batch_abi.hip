@@ -349,7 +349,8 @@ void enqueue_sort_and_forward(msplat_hip_ctx *ctx, BatchState *b, const msplat_h
     }
     // stably by view: each view's records in depth order, views in order
     launch_view_keys(dvi, &sc->nvis, R, g->num_points, dki, s);
-    launch_radix_pass(dki, dvi, dko, dvo, &sc->nvis, R, 0, (uint32_t *)b->hist.p, (uint32_t *)b->digit_total.p, s);
+    launch_radix_pass(dki, dvi, dko, dvo, &sc->nvis, R, 0, (uint32_t *)b->hist.p, (uint32_t *)b->digit_total.p, s, 0xFF,
+                      ListEntries{(const uint2 *)b->rect.p, (uint2 *)b->lrect.p, false});
     std::swap(dki, dko);
     std::swap(dvi, dvo);
     TileListArgs t;
@@ -357,8 +358,7 @@ void enqueue_sort_and_forward(msplat_hip_ctx *ctx, BatchState *b, const msplat_h
     t.list = dvi;
     t.nvis = &sc->nvis;
     t.overflow = &sc->overflow;
-    t.rect = (const uint2 *)b->rect.p;
-    t.lrect = (uint2 *)b->lrect.p;
+    t.lrect = (const uint2 *)b->lrect.p;
     t.coarse = (uint2 *)b->coarse.p;
     t.gids = (int32_t *)b->gids.p;
     t.tile_start = (int32_t *)b->tile_start.p;
@@ -392,7 +392,7 @@ void enqueue_backward(msplat_hip_ctx *ctx, BatchState *b, const msplat_hip_gauss
     float4 *ba = big_a(b);
     launch_big_reduce_records((const uint32_t *)b->big_list.p, &dsc(b)->big_count, (const uint32_t *)b->offsets.p,
                               (const uint32_t *)b->count.p, (const float4 *)b->slot_a.p, (const float4 *)b->slot_b.p,
-                              (const float *)b->slot_c.p, (const uint8_t *)b->slot_f.p, ba, ba + R, (float *)(ba + 2 * R), s);
+                              (const float *)b->slot_c.p, (const uint8_t *)b->slot_f.p, ba, ba + R, (float *)(ba + 2 * R), R, s);
     BatchBackwardArgs a;
     a.tab = dtab(b);
     a.n = g->num_points;

@@ -342,12 +342,17 @@ __global__ __launch_bounds__(256) void compact_kernel(CompactArgs a) {
 // intersections (in no particular order): each workgroup counts those of its part of the
 // records, takes its place in the list with one atomic, and writes them. One atomic per
 // 256 records, as the list was first built, serialised on its counter (about 12 ns each:
-// 21 us at 475k records, 360 us for a batch of 8 views of 1M).
-constexpr int SLOT_PREPARE_GRID = 1024;
+// 21 us at 475k records, 360 us for a batch of 8 views of 1M). 256 workgroups take 9.9 us
+// at 475k and 117 us for the batch, 1024 take 16.7 and 70.
+constexpr size_t SLOT_PREPARE_GRID = 1024;
+constexpr uint32_t SLOT_PREPARE_MANY = 2u << 20;
 __global__ __launch_bounds__(256) void slot_prepare_kernel(SlotPrepareArgs a) {
     __shared__ uint32_t lds4[4];
     __shared__ uint32_t s_base;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < a.nwords; i += (size_t)gridDim.x * 256) a.flag_words[i] = 0u;
+    const size_t tid = (size_t)blockIdx.x * 256 + threadIdx.x, quads = a.nwords / 4;
+    for (size_t i = tid; i < quads; i += (size_t)gridDim.x * 256)
+        reinterpret_cast<uint4 *>(a.flag_words)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < a.nwords - 4 * quads) a.flag_words[4 * quads + tid] = 0u;
     if (a.overflow && *a.overflow) return;
     const uint32_t per = (a.nrec + gridDim.x - 1) / gridDim.x;
     const uint32_t b = min(blockIdx.x * per, a.nrec), e = min(b + per, a.nrec);
@@ -437,7 +442,8 @@ __global__ __launch_bounds__(256) void rs_scan_kernel(uint32_t *hist, int stride
 // One element block of a pass; `my_base` is this thread's digit's global start for the block.
 template <typename K, int ITEMS>
 __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kout, int32_t *vout, uint32_t n,
-                                        int shift, uint32_t mask, uint32_t start, uint32_t my_base) {
+                                        int shift, uint32_t mask, uint32_t start, uint32_t my_base,
+                                        const ListEntries &entries) {
     constexpr int R = ITEMS / 256;  // rounds of 64 elements per wave
     __shared__ K sk[ITEMS];
     __shared__ int32_t sv[ITEMS];
@@ -505,6 +511,13 @@ __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kou
         const K k = sk[p];
         const uint32_t d = (uint32_t)(k >> shift) & mask;
         const uint32_t o = gbase[d] + (p - lstart[d]);
+        if (entries.lrect) {
+            const int32_t v = sv[p];
+            const uint2 q = entries.rect[v];
+            vout[o] = v;
+            entries.lrect[o] = entries.direct ? make_uint2((uint32_t)v, pack_local(q, 0, 0)) : q;
+            continue;
+        }
         kout[o] = k;
         if (has_vals) vout[o] = sv[p];
     }
@@ -514,7 +527,8 @@ __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kou
 template <typename K, int ITEMS>
 __global__ __launch_bounds__(256) void rs_scatter_kernel(const K *kin, const int32_t *vin, K *kout, int32_t *vout,
                                                         const uint32_t *n_ptr, int shift, uint32_t mask,
-                                                        const uint32_t *hist, int stride, const uint32_t *digit_total) {
+                                                        const uint32_t *hist, int stride, const uint32_t *digit_total,
+                                                        ListEntries entries) {
     __shared__ uint32_t dex[256];
     __shared__ uint32_t lds4[4];
     {   // exclusive prefix of the digit totals
@@ -525,7 +539,7 @@ __global__ __launch_bounds__(256) void rs_scatter_kernel(const K *kin, const int
     for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x) {
         __syncthreads();
         rs_scatter_block<K, ITEMS>(kin, vin, kout, vout, *n_ptr, shift, mask, b * ITEMS,
-                                   dex[threadIdx.x] + hist[(size_t)threadIdx.x * stride + b]);
+                                   dex[threadIdx.x] + hist[(size_t)threadIdx.x * stride + b], entries);
     }
 }
 
@@ -667,8 +681,9 @@ void launch_scan_blocks(uint32_t *sums, int nblocks, uint64_t *total, uint32_t *
 }
 
 void launch_slot_prepare(const SlotPrepareArgs &a, hipStream_t s) {
-    const size_t blocks = std::max((a.nwords + 255) / 256, ((size_t)a.nrec + 255) / 256);
-    if (blocks) slot_prepare_kernel<<<(unsigned)std::min<size_t>(blocks, SLOT_PREPARE_GRID), 256, 0, s>>>(a);
+    const size_t blocks = std::max((a.nwords + 1023) / 1024, ((size_t)a.nrec + 255) / 256);
+    const size_t most = a.nrec < SLOT_PREPARE_MANY ? SLOT_PREPARE_GRID / 4 : SLOT_PREPARE_GRID;
+    if (blocks) slot_prepare_kernel<<<(unsigned)std::min(blocks, most), 256, 0, s>>>(a);
 }
 
 void launch_compact(const CompactArgs &a, hipStream_t s) {
@@ -691,21 +706,25 @@ constexpr uint32_t HIST_GRID = 2048, SCATTER_GRID = 1024;
 template <typename K, int ITEMS>
 static void radix_pass_items(const K *kin, const int32_t *vin, K *kout, int32_t *vout, const uint32_t *n_dev,
                              uint32_t n_max, int shift, uint32_t mask, uint32_t *hist, uint32_t *digit_total,
-                             hipStream_t s) {
+                             hipStream_t s, const ListEntries &entries) {
     const uint32_t nblocks = (n_max + ITEMS - 1) / ITEMS;
     if (nblocks == 0) return;
     rs_hist_kernel<K, ITEMS><<<std::min(nblocks, HIST_GRID), 256, 0, s>>>(kin, n_dev, shift, mask, hist, (int)nblocks);
     rs_scan_kernel<ITEMS><<<256, 256, 0, s>>>(hist, (int)nblocks, n_dev, digit_total);
     rs_scatter_kernel<K, ITEMS><<<std::min(nblocks, SCATTER_GRID), 256, 0, s>>>(kin, vin, kout, vout, n_dev, shift,
-                                                                                mask, hist, (int)nblocks, digit_total);
+                                                                                mask, hist, (int)nblocks, digit_total,
+                                                                                entries);
 }
 
 template <typename K>
 static void radix_pass(const K *kin, const int32_t *vin, K *kout, int32_t *vout, const uint32_t *n_dev,
-                       uint32_t n_max, int shift, uint32_t mask, uint32_t *hist, uint32_t *digit_total, hipStream_t s) {
+                       uint32_t n_max, int shift, uint32_t mask, uint32_t *hist, uint32_t *digit_total, hipStream_t s,
+                       const ListEntries &entries = ListEntries{nullptr, nullptr, false}) {
     if (n_max >= RS_LARGE)
-        radix_pass_items<K, RS_ITEMS>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s);
-    else radix_pass_items<K, RS_ITEMS_SMALL>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s);
+        radix_pass_items<K, RS_ITEMS>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s, entries);
+    else
+        radix_pass_items<K, RS_ITEMS_SMALL>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s,
+                                            entries);
 }
 
 void launch_radix_pass(const uint64_t *kin, const int32_t *vin, uint64_t *kout, int32_t *vout, const uint32_t *n_dev,
@@ -714,8 +733,9 @@ void launch_radix_pass(const uint64_t *kin, const int32_t *vin, uint64_t *kout, 
 }
 
 void launch_radix_pass(const uint32_t *kin, const int32_t *vin, uint32_t *kout, int32_t *vout, const uint32_t *n_dev,
-                       uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s, uint32_t mask) {
-    radix_pass<uint32_t>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s);
+                       uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s, uint32_t mask,
+                       const ListEntries &entries) {
+    radix_pass<uint32_t>(kin, vin, kout, vout, n_dev, n_max, shift, mask, hist, digit_total, s, entries);
 }
 
 void launch_view_keys(const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n, uint32_t *keys,

@@ -161,6 +161,14 @@ __device__ inline float wave_sums10(const SumLanes &L, float q0, float q1, float
 
 __device__ inline uint64_t ballot(bool p) { return __ballot(p); }
 
+// A tile rectangle (x0 | x1 << 16, y0 | y1 << 16) within the supertile of 8x8 tiles at
+// (ox, oy): four 4-bit numbers x0 | x1 << 4 | y0 << 8 | y1 << 12
+__device__ inline uint32_t pack_local(uint2 r, int ox, int oy) {
+    const int x0 = min(max((int)(r.x & 0xFFFF) - ox, 0), 8), x1 = min(max((int)(r.x >> 16) - ox, 0), 8);
+    const int y0 = min(max((int)(r.y & 0xFFFF) - oy, 0), 8), y1 = min(max((int)(r.y >> 16) - oy, 0), 8);
+    return (uint32_t)(x0 | (x1 << 4) | (y0 << 8) | (y1 << 12));
+}
+
 // Orders LDS accesses of the lanes of one wave (no instruction is emitted).
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -90,8 +90,8 @@ struct TileListArgs {
     const int32_t *list;       // visible records, depth order (a batch: view after view)
     const uint32_t *nvis;      // device length of the list
     const uint32_t *overflow;  // null, or: when set the lists are empty
-    const uint2 *rect;         // per record
-    uint2 *lrect;              // scratch, one per list entry
+    // per list entry its record's rectangle, or with `direct` (record, pack_local)
+    const uint2 *lrect;
     uint2 *coarse;             // scratch: the supertiles' lists, at most one entry per intersection
     int32_t *gids;             // out: the tiles' lists
     int32_t *tile_start;       // out: list t is gids[tile_start[t], tile_start[t + 1])
@@ -404,7 +404,7 @@ void launch_batch_raster_backward(const BatchRasterArgs &a, const Tuning &t, hip
 void launch_batch_loss(const BatchLossArgs &a, hipStream_t s);
 void launch_big_reduce_records(const uint32_t *big_list, const uint32_t *big_count, const uint32_t *offsets,
                                const uint32_t *count, const float4 *slot_a, const float4 *slot_b, const float *slot_c,
-                               const uint8_t *slot_f, float4 *big_a, float4 *big_b, float *big_c, hipStream_t s);
+                               const uint8_t *slot_f, float4 *big_a, float4 *big_b, float *big_c, size_t nrec, hipStream_t s);
 void launch_batch_backward(const BatchBackwardArgs &a, hipStream_t s);
 // Adam over one parameter group from summed gradients; `vis` (per gaussian, null =
 // dense) restricts it to gaussians visible in some view, and for the SH rest group to
@@ -427,9 +427,16 @@ void launch_compact(const CompactArgs &a, hipStream_t s);
 void launch_radix_pass(const uint64_t *kin, const int32_t *vin, uint64_t *kout, int32_t *vout, const uint32_t *n_dev,
                        uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s,
                        uint32_t mask = 0xFF);
+// With entries, the pass is a last one: it writes no keys (kout may be null), and beside
+// each payload, a record, its tile list entry.
+struct ListEntries {
+    const uint2 *rect;  // per record
+    uint2 *lrect;       // out, TileListArgs::lrect; null: no entries
+    bool direct;
+};
 void launch_radix_pass(const uint32_t *kin, const int32_t *vin, uint32_t *kout, int32_t *vout, const uint32_t *n_dev,
                        uint32_t n_max, int shift, uint32_t *hist, uint32_t *digit_total, hipStream_t s,
-                       uint32_t mask = 0xFF);
+                       uint32_t mask = 0xFF, const ListEntries &entries = ListEntries{nullptr, nullptr, false});
 size_t radix_hist_words(uint32_t n_max);
 // batch: view ids of the depth-sorted records (record / n) as sort keys
 void launch_view_keys(const int32_t *recs, const uint32_t *n_dev, uint32_t n_max, int n, uint32_t *keys,

@@ -28,7 +28,8 @@
 //   20k, 128x128 (35k)                                33 ->  18 us
 // What bounds it: level 2's expansion by its stores (31 M words in 100 us at 1920x1080,
 // runs of about ten words), level 1's by the latency of its few waves; a small frame by
-// its launches (4-6 us each).
+// its launches (3-6 us each). The depth sort's last pass writes the first entries, in place of
+// a gather after it (per frame 4.7 us of launches for 3 of work at 475k, 7 less at 3M).
 #include <algorithm>
 
 #include "common.h"
@@ -234,8 +235,7 @@ __global__ __launch_bounds__(1024) void list_plan1_kernel(TileListArgs a) {
 // The supertiles' list starts and level-2 units from their totals (one workgroup).
 // plan[1] = the level-2 groups per unit.
 template <bool BATCH>
-__global__ __launch_bounds__(1024) void list_plan2_kernel(TileListArgs a) {
-    __shared__ uint32_t lds16[16];
+__device__ inline void plan2(const TileListArgs &a, uint32_t *lds16) {
     const uint32_t n = 64 * level1_nodes<BATCH>(a);
     uint32_t carry = 0;
     for (uint32_t b = 0; b < n; b += 1024) {
@@ -311,13 +311,8 @@ __device__ inline int tile_of(const TileListArgs &a, uint32_t i, int c) {
 
 // ── list entries ─────────────────────────────────────────────────────────────
 // A level-1 entry is a record and its tile rectangle; a level-2 entry is a record and the
-// rectangle within its supertile, four 4-bit numbers x0 | x1 << 4 | y0 << 8 | y1 << 12.
-__device__ inline uint32_t pack_local(uint2 r, int ox, int oy) {
-    const int x0 = min(max((int)(r.x & 0xFFFF) - ox, 0), 8), x1 = min(max((int)(r.x >> 16) - ox, 0), 8);
-    const int y0 = min(max((int)(r.y & 0xFFFF) - oy, 0), 8), y1 = min(max((int)(r.y >> 16) - oy, 0), 8);
-    return (uint32_t)(x0 | (x1 << 4) | (y0 << 8) | (y1 << 12));
-}
-
+// rectangle within its supertile (pack_local). The last pass of the depth sort writes the
+// first entries (level 1 reads them once per node) beside the records.
 __device__ inline void local_mask(uint32_t p, uint32_t &lo, uint32_t &hi) {
     cell_mask((int)(p & 15), (int)((p >> 4) & 15), (int)((p >> 8) & 15), (int)((p >> 12) & 15), lo, hi);
 }
@@ -327,17 +322,6 @@ __device__ inline void super_mask(uint2 r, int hx, int hy, uint32_t &lo, uint32_
     const int x0 = (int)((r.x & 0xFFFF) >> 3) - 8 * hx, x1 = (int)(((r.x >> 16) + 7) >> 3) - 8 * hx;
     const int y0 = (int)((r.y & 0xFFFF) >> 3) - 8 * hy, y1 = (int)(((r.y >> 16) + 7) >> 3) - 8 * hy;
     cell_mask(max(x0, 0), min(x1, 8), max(y0, 0), min(y1, 8), lo, hi);
-}
-
-// The rectangles in list order (level 1 reads them once per node), or, for a view of one
-// supertile, its level-2 entries
-__global__ __launch_bounds__(256) void list_gather_kernel(TileListArgs a) {
-    const uint32_t nvis = visible(a);
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < nvis; i += gridDim.x * 256) {
-        const int32_t r = a.list[i];
-        const uint2 q = a.rect[r];
-        a.lrect[i] = a.direct ? make_uint2((uint32_t)r, pack_local(q, 0, 0)) : q;
-    }
 }
 
 // ── level 1: the records of a wave's part that touch the node ────────────────
@@ -525,6 +509,29 @@ __global__ __launch_bounds__(64 * PREFIX_WAVES) void list_prefix1_kernel(TileLis
     }
 }
 
+template <bool BATCH>
+__global__ __launch_bounds__(1024) void list_plan2_kernel(TileListArgs a) {
+    __shared__ uint32_t lds16[16];
+    plan2<BATCH>(a, lds16);
+}
+
+// Both for a view of few nodes, in one workgroup: 7.7 us for 9.5 at one and two nodes, but
+// 11.6 for 9.4 at four.
+constexpr uint32_t FEW_NODES = 2;
+static_assert(64 * PREFIX_WAVES == 1024, "one workgroup shape");
+__global__ __launch_bounds__(1024) void list_prefix1_plan2_kernel(TileListArgs a) {
+    __shared__ uint32_t sums[PREFIX_WAVES][64];
+    __shared__ uint32_t lds16[16];
+    for (uint32_t i = 0; i < (uint32_t)a.nodes; i++) {
+        const Node1 k = level1_node<false>(a, i);
+        const uint32_t units = unit_count<WAVES1>(k.e - k.s, k.groups);
+        const uint32_t t = prefix_rows<PREFIX_WAVES>(a.cnt1, k.first_unit, k.first_unit + units, sums);
+        if (threadIdx.x < 64) a.super_total[64 * i + threadIdx.x] = t;
+    }
+    __syncthreads();  // the totals, which other threads of the workgroup read
+    plan2<false>(a, lds16);
+}
+
 // Level 2: a tile's total goes to tile_start[tile], to be scanned in tile order
 template <bool BATCH>
 __global__ __launch_bounds__(64 * PREFIX_WAVES) void list_prefix2_kernel(TileListArgs a) {
@@ -685,11 +692,13 @@ static uint32_t unit_blocks(uint64_t entries, uint32_t nodes) {
 
 template <bool BATCH>
 static void lists_begin(const TileListArgs &a, uint32_t nodes, uint32_t nvis_max, hipStream_t s) {
-    const uint32_t list_blocks = (nvis_max + 255) / 256;
-    if (list_blocks) list_gather_kernel<<<list_blocks < 2048 ? list_blocks : 2048, 256, 0, s>>>(a);
     if (a.direct) return;
     if (BATCH) list_plan1_kernel<<<1, 1024, 0, s>>>(a);
     list_count1_kernel<BATCH><<<unit_blocks<WAVES1>((uint64_t)nodes * nvis_max, nodes), 64 * WAVES1, 0, s>>>(a);
+    if (!BATCH && nodes <= FEW_NODES) {
+        list_prefix1_plan2_kernel<<<1, 1024, 0, s>>>(a);
+        return;
+    }
     list_prefix1_kernel<BATCH><<<nodes < 1024 ? nodes : 1024, 64 * PREFIX_WAVES, 0, s>>>(a);
     list_plan2_kernel<BATCH><<<1, 1024, 0, s>>>(a);
 }

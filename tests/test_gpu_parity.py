@@ -273,6 +273,41 @@ def test_backward_gradients_match_oracle(ctx, oracle, ppt):
         ctx.set_tuning(TUNE_BWD_PPT, default_ppt)
 
 
+@pytest.mark.parametrize("W,H", [(512, 512), (530, 513)])
+def test_slot_sums_of_records_over_many_tiles(ctx, oracle, W, H):
+    """Gaussians of up to every tile of the view, more than one wave's 1020 slots (the first
+    six, of which a workgroup sets two aside and sums the others in place), beside ones of
+    33 to 1020 and fewer than 33. Against the oracle's in-order sums: the per-record
+    gradients differ by the pairs' own errors and by a sum of at most 1100 terms in another
+    order, 1100 * 6e-8 = 7e-5 of the terms' absolute sum at worst."""
+    from msplat._abi import DeviceArray, FRAME_KEEP_GRADS
+    from msplat.backend import DeviceGaussians, render, render_backward
+    from msplat.scenes import random_scene
+    sc, cam = _scene_cam(seed=41, n=60, deg=1, W=W, H=H)
+    sc["opac"][:] = -3.0  # every record reaches the pixels behind it
+    sc["scales"][:] = np.random.default_rng(42).uniform(-4.5, 1.0, (60, 1)).astype(np.float32)
+    sc["means"][:6] *= 0.1
+    sc["scales"][:6] = np.array([2.5, 2.4, 2.6, 2.7, 2.45, 2.55], np.float32)[:, None]
+    dg = DeviceGaussians(ctx, sc)
+    v_img = (np.random.default_rng(43).normal(0, 1, (H, W, 3)) * 1e-3).astype(np.float32)
+    ctx.set_flags(FRAME_KEEP_GRADS)
+    try:
+        render(ctx, dg, cam, BG)
+        render_backward(ctx, dg, cam, BG, DeviceArray.from_numpy(ctx, v_img))
+        f = ctx.frame()
+        got = dict(v_xy=ctx.download(f.v_xy, (60, 2), np.float32), v_conic=ctx.download(f.v_conic, (60, 3), np.float32),
+                   v_rgb=ctx.download(f.v_rgb, (60, 3), np.float32), v_opac=ctx.download(f.v_opacity, (60,), np.float32))
+        _, b, fwd = oracle.render(sc, cam, BG)
+        slots = oracle.raster_backward(b, fwd, cam, BG, v_img)
+        red = oracle.reduce_slots(60, b, slots)
+        count = np.bincount(ctx.download(f.isect_gid, (int(f.num_isects),), np.int32), minlength=60)
+        assert (count[:6] > 1020).all() and ((count > 32) & (count <= 1020)).any() and (count[count > 0] <= 32).any()
+        for k in got:
+            assert _rel(got[k], red[k].reshape(got[k].shape)) < 1e-4, k
+    finally:
+        ctx.set_flags(0)
+
+
 def test_train_steps_match_golden(ctx):
     """Three GPU train steps against the reference's own three steps (golden vectors)."""
     from msplat._abi import DeviceArray

@@ -40,6 +40,7 @@ def _expected(ctx, f, n, tiles_x, tiles_y):
     (1024, 1024, 500, -2.5),  # exactly one level-1 node
     (1025, 1040, 500, -1.5),  # four nodes, three of them one tile wide
     (2070, 40, 400, -2.0),    # three nodes side by side
+    (1030, 2060, 400, -2.0),  # six nodes: the first launches of their own for prefix and plan
     (640, 360, 5000, -4.0),   # several units per node
     (200, 150, 70000, -5.0),  # more entries than one group per wave holds at level 2
 ])
@@ -93,3 +94,38 @@ def test_batched_lists_give_the_one_view_images(graph):
             np.testing.assert_array_equal(img, render_numpy(one, dg, c, BG))
     ctx.close()
     one.close()
+
+
+def _one_tile_cloud(n):
+    """Depths over three octaves and many ties; some gaussians behind the camera."""
+    from msplat.scenes import random_scene
+    rng = np.random.default_rng(n)
+    sc = random_scene(n, n, degree=0, log_scale=(-3.0, 0.1))
+    sc["means"] = (rng.normal(0, 0.02, (n, 3))).astype(np.float32)
+    z = rng.uniform(-0.5, 9, n).astype(np.float32)
+    z[n // 2:] = np.round(z[n // 2:], 2)  # equal depths: the id breaks the tie
+    sc["means"][:, 2] += z
+    return sc
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 300_000, 2 << 20])
+def test_depth_order_at_block_edges(n):
+    """One tile holds every visible gaussian, in (depth bits, id) order: around one block of
+    the sort, whose last pass writes the list entries, and with its larger blocks."""
+    from msplat._abi import Context
+    from msplat.backend import DeviceGaussians, render
+    from msplat.camera import look_at, make_camera
+    ctx = Context(0)
+    cam = make_camera(look_at((0, 0, -1), (0, 0, 1)), 16, 16, 14.0, 14.0)
+    dg = DeviceGaussians(ctx, _one_tile_cloud(n))
+    for _ in range(2):
+        render(ctx, dg, cam, BG)
+        f = ctx.frame()
+        rad, dep = ctx.download(f.radii, (n,), np.int32), ctx.download(f.depths, (n,), np.float32)
+        c = ctx.download(f.splat_a, (n, 4), np.float32)[:, :2] / np.float32(16)
+        r = ctx.download(f.aabb, (n, 2), np.float32) / np.float32(16)
+        ids = np.nonzero((rad > 0) & np.all((c - r < 1) & (c + r + np.float32(1) >= 1), axis=1))[0]
+        gids = ctx.download(f.isect_gid, (int(f.num_isects),), np.int32)
+        np.testing.assert_array_equal(gids, ids[np.lexsort((ids, dep[ids].view(np.uint32)))])
+    assert n == 1 or len(gids) > 0.8 * n
+    ctx.close()
