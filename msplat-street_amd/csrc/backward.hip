@@ -488,7 +488,9 @@ constexpr int SH_ADAM_GRID = 4096;
 // the views and taken through the covariance VJP once (it is linear in them), and the
 // SH band cotangents basis(dir_v) x v_rgb_v are summed per coefficient. The
 // densification statistics are updated per view as a sequence of one-view steps would.
-__global__ __launch_bounds__(256) void batch_backward_kernel(BatchBackwardArgs a) {
+// Bound by the latency of its dependent loads: three waves per SIMD (168 registers, five
+// spilled) take 432 us for 8 views of 1M gaussians, two (172 registers) 482, four 580.
+__global__ __launch_bounds__(256, 3) void batch_backward_kernel(BatchBackwardArgs a) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (g >= a.n || a.sc->overflow) return;
     const float p[3] = {a.means[3 * g], a.means[3 * g + 1], a.means[3 * g + 2]};

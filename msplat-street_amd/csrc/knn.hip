@@ -15,7 +15,7 @@
 // What bounds it: the scalar steps of a wave (a leaf visited, a query taken) and the latency
 // of its dependent loads. A leaf of 64 is what one wave holds as queries and as candidates.
 // It replaced one thread per query walking boxes of 128 points, whose 64 lanes disagreed on
-// almost every box: the 475k points of a street, 2300 -> 240 us (a whole initialisation, 2450
+// almost every box: the 475k points of a street, 2300 -> 280 us (a whole initialisation, 2450
 // -> 390 us); 20k points, 1318 -> 243 us with the ordering; 200k points in one cell of the
 // curve, beside an outlier at a thousand times their extent, 26.7 -> 3.6 ms.
 #include "common.h"
