@@ -321,8 +321,11 @@ __device__ inline uint32_t sum_written(const BackwardArgs &a, uint32_t o, uint32
 // is written), one wave each, grid-stride over the device-side list; the nine lane sums
 // (ten with depth slots) are added over the wave by wave_sums9 (wave_sums10). The next
 // record's flags are loaded while this one's values are on their way, and its id and slot
-// range a record earlier. Records of more than BR_SLOTS slots, up to every tile of the view,
-// are left to the end, where the workgroup's waves sum BR_SLOTS slots of one each in turn.
+// range a record earlier. A record of more than BR_SLOTS slots, up to every tile of the view,
+// is the sum in order of four parts, part k being its chunks of BR_SLOTS slots k, k + 4, ...:
+// the first few that a workgroup meets are left to the end, where each wave sums one part; any
+// others are summed part after part where they are met. Which way a record goes depends on the
+// order of the list (built by racing workgroups); its sum, bit for bit, does not.
 //
 // Bound by the round trips of a record (flags, then values) and by the largest records.
 // Reading all slots' flags byte by byte and the written values four strided slots at a time,
@@ -353,6 +356,16 @@ __global__ __launch_bounds__(256) void big_reduce_kernel(BackwardArgs a) {
         return a.slot_d ? wave_sums10(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9])
                         : wave_sums9(sl, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]);
     };
+    // part k of the c > BR_SLOTS slots from o
+    auto part_sums = [&](uint32_t o, uint32_t c, uint32_t k) {
+        float v[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        uint32_t fp[BR_ROUNDS];
+        for (uint32_t s = k * BR_SLOTS; s < c; s += 4 * BR_SLOTS) {
+            load_flags(a.slot_f, o + s, min(c - s, BR_SLOTS), lane, fp);
+            sum_written(a, o + s, min(c - s, BR_SLOTS), fp, list, lane, v, [] {});
+        }
+        return sums(v);
+    };
     auto store = [&](uint32_t g, float t) {
         if (a.slot_d && lane == 9) a.big_d[g] = t;
         if (lane < 9) {
@@ -378,19 +391,19 @@ __global__ __launch_bounds__(256) void big_reduce_kernel(BackwardArgs a) {
         }
         if (at < BR_HUGE) {
             load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
+        } else if (c > BR_SLOTS) {
+            float t = part_sums(o, c, 0);
+            for (uint32_t k = 1; k < 4; k++) t += part_sums(o, c, k);
+            store(g, t);
+            load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
         } else {
             float v[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            uint32_t written = 0;
-            for (uint32_t s = 0; s < c; s += BR_SLOTS) {  // the next flags: this record's, or the next one's
-                const bool more = s + BR_SLOTS < c;
-                uint32_t fc[BR_ROUNDS];
+            uint32_t fc[BR_ROUNDS];
 #pragma unroll
-                for (int r = 0; r < BR_ROUNDS; r++) fc[r] = f[r];
-                written += sum_written(a, o + s, min(c - s, BR_SLOTS), fc, list, lane, v, [&] {
-                    if (more) load_flags(a.slot_f, o + s + BR_SLOTS, min(c - s - BR_SLOTS, BR_SLOTS), lane, f);
-                    else load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
-                });
-            }
+            for (int r = 0; r < BR_ROUNDS; r++) fc[r] = f[r];
+            const uint32_t written = sum_written(a, o, c, fc, list, lane, v, [&] {
+                load_flags(a.slot_f, on, min(cn, BR_SLOTS), lane, f);
+            });
             store(g, written ? sums(v) : 0.f);
         }
         g = gn; o = on; c = cn;
@@ -400,13 +413,8 @@ __global__ __launch_bounds__(256) void big_reduce_kernel(BackwardArgs a) {
     __syncthreads();
     const uint32_t nh = min(nhuge, BR_HUGE);
     for (uint32_t k = 0; k < nh; k++) {
-        const uint32_t h = scalar(huge[k]), ho = scalar(a.offsets[h]), hc = scalar(a.count[h]);
-        float v[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (uint32_t s = w * BR_SLOTS; s < hc; s += 4 * BR_SLOTS) {
-            load_flags(a.slot_f, ho + s, min(hc - s, BR_SLOTS), lane, f);
-            sum_written(a, ho + s, min(hc - s, BR_SLOTS), f, list, lane, v, [] {});
-        }
-        const float t = sums(v);
+        const uint32_t h = scalar(huge[k]);
+        const float t = part_sums(scalar(a.offsets[h]), scalar(a.count[h]), (uint32_t)w);
         if (lane < 9) part[w][sl.q] = t;
         if (lane == 9) part[w][9] = t;
         __syncthreads();

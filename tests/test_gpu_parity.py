@@ -308,6 +308,72 @@ def test_slot_sums_of_records_over_many_tiles(ctx, oracle, W, H):
         ctx.set_flags(0)
 
 
+def _many_large_records(n=200, large=48, W=1040, H=1040):
+    """A view whose first `large` records cover most or all of its 4225 tiles (more than four
+    waves' 1020 slots each), far more of them than the slot sums' workgroups set aside."""
+    sc, cam = _scene_cam(seed=45, n=n, deg=1, W=W, H=H)
+    rng = np.random.default_rng(46)
+    sc["opac"][:] = -4.0  # every record reaches the pixels behind it
+    sc["scales"][:large] = rng.uniform(2.3, 2.8, (large, 1)).astype(np.float32)
+    sc["means"][:large] *= 0.1
+    return sc, cam, (rng.normal(0, 1, (H, W, 3)) * 1e-3).astype(np.float32)
+
+
+def test_slot_sums_of_large_records_repeat_exactly(ctx):
+    """Every backward of one frame, and of the same frame rendered again, gives the same bits
+    whichever order the records are listed in (the list is built by racing workgroups)."""
+    from msplat._abi import DeviceArray
+    from msplat.backend import DeviceGaussians, render, render_backward
+    sc, cam, v = _many_large_records()
+    dg, v_img = DeviceGaussians(ctx, sc), DeviceArray.from_numpy(ctx, v)
+    ref = None
+    for _ in range(3):
+        render(ctx, dg, cam, BG)
+        f = ctx.frame()
+        count = np.bincount(ctx.download(f.isect_gid, (int(f.num_isects),), np.int32), minlength=dg.n)
+        assert (count > 1020).sum() >= 48
+        for _ in range(4):
+            got = render_backward(ctx, dg, cam, BG, v_img)
+            ref = ref or got
+            for k in ref:
+                assert np.abs(ref[k]).max() > 0, k
+                np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+def test_slot_sums_of_large_records_in_a_batch(ctx):
+    """The same through a batch of two views: repeated exactly, and equal to the one-view
+    gradients' sum (each record's slot sums are the one-view ones; the two views' vector-
+    Jacobian products add in another order, a few roundings of 6e-8 of the largest)."""
+    from msplat._abi import TUNE_CHUNKS, DeviceArray
+    from msplat.backend import BatchViews, DeviceGaussians, render, render_backward, render_backward_batch, render_batch
+    sc, cam, v = _many_large_records()
+    cams = [cam, dict(_scene_cam(seed=45, n=1, deg=1, W=1040, H=560)[1], dtu=1)]
+    vs = [v, np.ascontiguousarray(v[:560] * np.float32(0.5))]
+    dg = DeviceGaussians(ctx, sc)
+    bv = BatchViews(cams, 1, [BG])
+    total = {}
+    saved = ctx.get_tuning(TUNE_CHUNKS)
+    ctx.set_tuning(TUNE_CHUNKS, 1)  # the batched rasterizer's per-tile form
+    try:
+        for c, x in zip(cams, vs):
+            render(ctx, dg, c, BG)
+            for k, g in render_backward(ctx, dg, c, BG, DeviceArray.from_numpy(ctx, x)).items():
+                total[k] = total.get(k, 0) + g.astype(np.float64)
+    finally:
+        ctx.set_tuning(TUNE_CHUNKS, saved)
+    packed = DeviceArray.from_numpy(ctx, np.concatenate([x.reshape(-1, 3) for x in vs]))
+    ref = None
+    for _ in range(2):
+        render_batch(ctx, dg, bv)
+        for _ in range(4):
+            got = render_backward_batch(ctx, dg, bv, packed)
+            ref = ref or got
+            for k in ref:
+                np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+    for k in total:
+        assert np.abs(got[k] - total[k]).max() <= 2e-5 * np.abs(total[k]).max(), k
+
+
 def test_train_steps_match_golden(ctx):
     """Three GPU train steps against the reference's own three steps (golden vectors)."""
     from msplat._abi import DeviceArray

@@ -98,6 +98,39 @@ def test_prior_steps_with_a_full_sky_texture_match_oracle(ctx, oracle):
         assert v < 1e-4, (k, v)
 
 
+def test_depth_slots_of_large_records(ctx, oracle):
+    """Records over more than 1020 tiles, far more of them than the slot sums' workgroups set
+    aside, with depth slots: the same bits from every run of a step, and the oracle's sums
+    within the 1e-4 of the tests above."""
+    from msplat._abi import DeviceArray
+    from msplat.backend import DeviceGaussians
+    from msplat.prior import DevicePrior, train_step_prior
+    W, H, n, large = 560, 544, 160, 40  # 1190 tiles
+    sc, cam, gt, prior = prior_workload(seed=9, n=n, W=W, H=H, features=("aux", "depth"))
+    rng = np.random.default_rng(10)
+    sc["opac"][:] = -4.0
+    sc["scales"][:large] = rng.uniform(2.3, 2.8, (large, 1)).astype(np.float32)
+    sc["means"][:large] *= 0.1
+    gt_d = DeviceArray.from_numpy(ctx, gt)
+    ref = None
+    for _ in range(5):
+        dg = DeviceGaussians(ctx, sc)
+        train_step_prior(ctx, dg, cam, BG, gt_d, STEPS, BC2, DevicePrior(ctx, prior))
+        got = dg.to_numpy()
+        ref = ref or got
+        for k in KEYS:
+            for pre in ("", "m1_", "m2_"):
+                np.testing.assert_array_equal(got[pre + k], ref[pre + k], err_msg=pre + k)
+    f = ctx.frame()
+    count = np.bincount(ctx.download(f.isect_gid, (int(f.num_isects),), np.int32), minlength=n)
+    assert (count > 1020).sum() >= large
+    st = _state(sc)
+    oracle.train_step_prior(st, cam, BG, gt, STEPS, BC2, prior)
+    for k in KEYS:
+        for pre in ("", "m1_", "m2_"):
+            assert _rel(ref[pre + k], st[pre + k].reshape(ref[pre + k].shape)) < 1e-4, pre + k
+
+
 @pytest.mark.parametrize("variant", ["all", "aux_sky", "aux_defaults"])
 def test_prior_render_matches_oracle(ctx, oracle, variant):
     from msplat.backend import DeviceGaussians
