@@ -341,37 +341,31 @@ def test_slot_sums_of_large_records_repeat_exactly(ctx):
 
 
 def test_slot_sums_of_large_records_in_a_batch(ctx):
-    """The same through a batch of two views: repeated exactly, and equal to the one-view
-    gradients' sum (each record's slot sums are the one-view ones; the two views' vector-
-    Jacobian products add in another order, a few roundings of 6e-8 of the largest)."""
+    """The same through batches: a batch of one view gives the one-view gradients bit for bit,
+    a batch of two views the same bits every time."""
     from msplat._abi import TUNE_CHUNKS, DeviceArray
     from msplat.backend import BatchViews, DeviceGaussians, render, render_backward, render_backward_batch, render_batch
     sc, cam, v = _many_large_records()
-    cams = [cam, dict(_scene_cam(seed=45, n=1, deg=1, W=1040, H=560)[1], dtu=1)]
+    cams = [cam, _scene_cam(seed=45, n=1, deg=1, W=1040, H=560)[1]]
     vs = [v, np.ascontiguousarray(v[:560] * np.float32(0.5))]
     dg = DeviceGaussians(ctx, sc)
-    bv = BatchViews(cams, 1, [BG])
-    total = {}
     saved = ctx.get_tuning(TUNE_CHUNKS)
     ctx.set_tuning(TUNE_CHUNKS, 1)  # the batched rasterizer's per-tile form
     try:
-        for c, x in zip(cams, vs):
-            render(ctx, dg, c, BG)
-            for k, g in render_backward(ctx, dg, c, BG, DeviceArray.from_numpy(ctx, x)).items():
-                total[k] = total.get(k, 0) + g.astype(np.float64)
+        render(ctx, dg, cam, BG)
+        one = render_backward(ctx, dg, cam, BG, DeviceArray.from_numpy(ctx, v))
     finally:
         ctx.set_tuning(TUNE_CHUNKS, saved)
-    packed = DeviceArray.from_numpy(ctx, np.concatenate([x.reshape(-1, 3) for x in vs]))
-    ref = None
-    for _ in range(2):
-        render_batch(ctx, dg, bv)
-        for _ in range(4):
-            got = render_backward_batch(ctx, dg, bv, packed)
-            ref = ref or got
-            for k in ref:
-                np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
-    for k in total:
-        assert np.abs(got[k] - total[k]).max() <= 2e-5 * np.abs(total[k]).max(), k
+    for views, ref in ((1, one), (2, None)):
+        bv = BatchViews(cams[:views], 1, [BG])
+        packed = DeviceArray.from_numpy(ctx, np.concatenate([x.reshape(-1, 3) for x in vs[:views]]))
+        for _ in range(2):
+            render_batch(ctx, dg, bv)
+            for _ in range(4):
+                got = render_backward_batch(ctx, dg, bv, packed)
+                ref = ref or got
+                for k in ref:
+                    np.testing.assert_array_equal(got[k], ref[k], err_msg=f"{views} views, {k}")
 
 
 def test_train_steps_match_golden(ctx):
