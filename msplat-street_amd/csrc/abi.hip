@@ -36,6 +36,7 @@ namespace {
 int do_project(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, const msplat_hip_camera *cam,
                const StepParams *sp = nullptr) {
     ctx->frame_aux = false;  // a prior-guided entry point sets it after the projection
+    ctx->frame_stage = msplat_hip_ctx::FRAME_NONE;  // the last frame's buffers are rewritten, or moved, below
     const int n = g->num_points;
     const size_t N = (size_t)(n > 0 ? n : 1);
     const int nblocks = (n + 255) / 256;
@@ -1119,10 +1120,12 @@ int msplat_hip_frame_view(msplat_hip_ctx *ctx, msplat_hip_frame *f) {
     f->tile_count = (uint32_t *)ctx->count.p;
     f->offsets = (uint32_t *)ctx->offsets.p;
     f->isect_keys = nullptr;
-    f->isect_gid = ctx->gid_sorted;
-    if ((ctx->flags & MSPLAT_FRAME_KEYS64) && ctx->gid_sorted) {
+    // the lists belong to a binned frame: before that, gid_sorted and tile_start are an earlier one's
+    const bool binned = ctx->frame_stage >= msplat_hip_ctx::FRAME_BINNED;
+    f->isect_gid = binned ? ctx->gid_sorted : nullptr;
+    if ((ctx->flags & MSPLAT_FRAME_KEYS64) && binned) {
         CHECKED(ctx->grow(ctx->keys64, 8 * (size_t)(ctx->M > 0 ? ctx->M : 1)));
-        launch_list_keys64((const int32_t *)ctx->tile_start.p, ctx->ntiles, ctx->gid_sorted,
+        launch_list_keys64((const int32_t *)ctx->tile_start.p, ctx->ntiles, (int)ctx->M, ctx->gid_sorted,
                            (const float *)ctx->depths.p, (uint64_t *)ctx->keys64.p, ctx->stream);
         HIPCHECK(hipGetLastError());
         f->isect_keys = (uint64_t *)ctx->keys64.p;
@@ -1179,7 +1182,6 @@ int msplat_hip_radix_sort(msplat_hip_ctx *ctx, uint64_t *keys, int32_t *vals, ui
     }
     HIPCHECK(hipGetLastError());
     // the call ends the frame in the workspace: its lists are no longer offered
-    ctx->gid_sorted = nullptr;
     if (ctx->frame_stage > msplat_hip_ctx::FRAME_PROJECTED) ctx->frame_stage = msplat_hip_ctx::FRAME_PROJECTED;
     return MSPLAT_OK;
 }

@@ -112,7 +112,7 @@ void tile_list_carve(uint32_t *scratch, uint32_t nodes, TileListArgs &a);
 void launch_tile_lists_begin(const TileListArgs &a, bool batch, uint32_t nodes, uint32_t nvis_max, hipStream_t s);
 void launch_tile_lists_end(const TileListArgs &a, bool batch, uint32_t nodes, uint32_t nvis_max, uint32_t m_max,
                            uint32_t ntiles, uint32_t *partial, hipStream_t s);
-void launch_list_keys64(const int32_t *tile_start, int ntiles, const int32_t *gid, const float *depths, uint64_t *out,
+void launch_list_keys64(const int32_t *tile_start, int ntiles, int m, const int32_t *gid, const float *depths, uint64_t *out,
                         hipStream_t s);
 
 struct RasterArgs {

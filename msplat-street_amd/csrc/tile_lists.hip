@@ -647,11 +647,12 @@ __global__ __launch_bounds__(64 * WAVES2) void list_expand2_kernel(TileListArgs 
     }
 }
 
-// The 64-bit (tile << 32 | depth bits) view of the lists, one workgroup per tile
-__global__ __launch_bounds__(256) void list_keys64_kernel(const int32_t *tile_start, const int32_t *gid,
+// The 64-bit (tile << 32 | depth bits) view of the m listed intersections, one workgroup per tile
+__global__ __launch_bounds__(256) void list_keys64_kernel(const int32_t *tile_start, int m, const int32_t *gid,
                                                          const float *depths, uint64_t *out) {
     const uint32_t t = blockIdx.x;
-    for (int k = tile_start[t] + (int)threadIdx.x; k < tile_start[t + 1]; k += 256)
+    const int e = min(tile_start[t + 1], m);
+    for (int k = tile_start[t] + (int)threadIdx.x; k < e; k += 256)
         out[k] = ((uint64_t)t << 32) | (uint64_t)__float_as_uint(depths[gid[k]]);
 }
 
@@ -728,9 +729,9 @@ void launch_tile_lists_end(const TileListArgs &a, bool batch, uint32_t nodes, ui
     else lists_end<false>(a, nodes, nvis_max, m_max, ntiles, partial, s);
 }
 
-void launch_list_keys64(const int32_t *tile_start, int ntiles, const int32_t *gid, const float *depths, uint64_t *out,
+void launch_list_keys64(const int32_t *tile_start, int ntiles, int m, const int32_t *gid, const float *depths, uint64_t *out,
                         hipStream_t s) {
-    if (ntiles > 0) list_keys64_kernel<<<ntiles, 256, 0, s>>>(tile_start, gid, depths, out);
+    if (ntiles > 0) list_keys64_kernel<<<ntiles, 256, 0, s>>>(tile_start, m, gid, depths, out);
 }
 
 }  // namespace msplat

@@ -69,3 +69,41 @@ def test_out_of_order_stages_are_refused():
         ctx.sync()
     finally:
         ctx.close()
+
+
+def test_lists_are_offered_for_a_binned_frame_only():
+    """A frame that is projected, or whose radix sort ended it, has no lists: the earlier
+    frame's ids and ranges are not offered, nor read for the 64-bit keys of the new one's
+    tiles. Binned, they are the new frame's."""
+    from msplat._abi import FRAME_KEYS64, Context, DeviceArray, check, lib, make_camera_struct
+    from msplat.backend import DeviceGaussians, render_numpy
+    from msplat.camera import look_at, make_camera
+    sc, small = _scene()
+    large = make_camera(look_at((2.5, 0.7, 2.9), (0.1, -0.2, 0)), 320, 240, 300.0, 300.0, dtu=1)
+    ctx = Context(0)
+    try:
+        dg, L = DeviceGaussians(ctx, sc), lib()
+        ctx.set_flags(FRAME_KEYS64)
+        render_numpy(ctx, dg, small, BG)
+        assert ctx.frame().isect_gid and ctx.frame().isect_keys
+        g, c = dg.struct(), make_camera_struct(large, 1)
+        check(L.msplat_hip_stage_project(ctx.ptr, C.byref(g), C.byref(c)))
+        f = ctx.frame()
+        assert f.num_tiles == 20 * 15 and not f.isect_gid and not f.isect_keys
+        check(L.msplat_hip_stage_bin(ctx.ptr, C.byref(c)))
+        f = ctx.frame()
+        M = int(f.num_isects)
+        start = ctx.download(f.tile_start, (f.num_tiles + 1,), np.int32)
+        keys = ctx.download(f.isect_keys, (M,), np.uint64)
+        assert start[-1] == M > 0
+        np.testing.assert_array_equal(keys >> np.uint64(32), np.repeat(np.arange(f.num_tiles), np.diff(start)))
+        depths = ctx.download(f.depths, (dg.n,), np.float32)
+        np.testing.assert_array_equal((keys & np.uint64(0xFFFFFFFF)).astype(np.uint32),
+                                      depths[ctx.download(f.isect_gid, (M,), np.int32)].view(np.uint32))
+        sorted_keys = DeviceArray.from_numpy(ctx, np.arange(100, 0, -1, dtype=np.uint64))
+        vals = DeviceArray.from_numpy(ctx, np.arange(100, dtype=np.int32))
+        check(L.msplat_hip_radix_sort(ctx.ptr, C.c_void_p(sorted_keys.ptr), C.c_void_p(vals.ptr), 100, 32))
+        f = ctx.frame()
+        assert not f.isect_gid and not f.isect_keys
+    finally:
+        ctx.close()
