@@ -82,3 +82,39 @@ def test_a_pixel_without_a_finite_gradient_spares_what_it_does_not_see():
         assert far.sum() > 200 and np.isfinite(g[far]).all()
         assert not np.isfinite(g[~far]).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("chunks", [1, 3])
+def test_an_opacity_that_is_not_a_number(oracle, chunks):
+    """min(0.999, NaN) is 0.999, in the reference and here: such a record composites as an
+    opaque one, and every gradient but its own opacity's is finite."""
+    from msplat._abi import FRAME_KEEP_GRADS, TUNE_CHUNKS, Context, DeviceArray
+    from msplat.backend import DeviceGaussians, render, render_backward
+    from msplat.camera import look_at, make_camera
+    from msplat.scenes import random_scene
+    n, W, H = 600, 97, 71
+    sc = random_scene(23, n, degree=0, log_scale=(-3.4, 0.3), opac=(-1.0, 1.0))
+    sc["opac"][::15] = np.nan
+    cam = make_camera(look_at((2.2, 0.4, 2.6), (0, 0, 0)), W, H, 90.0, 88.0)
+    ctx = Context(0)
+    ctx.set_tuning(TUNE_CHUNKS, chunks)
+    ctx.set_flags(FRAME_KEEP_GRADS)
+    dg = DeviceGaussians(ctx, sc)
+    img = ctx.download(render(ctx, dg, cam, BG), (H, W, 3), np.float32)
+    p, b, fwd = oracle.render(sc, cam, BG)
+    assert _rel(img, fwd["img"]) < 1e-5
+    f = ctx.frame()
+    last = ctx.download(f.final_idx, (H, W), np.int32)
+    assert np.mean(last == fwd["final_idx"].reshape(H, W)) > 0.998
+    v_img = (np.random.default_rng(9).normal(0, 1, (H, W, 3)) * 1e-3).astype(np.float32)
+    render_backward(ctx, dg, cam, BG, DeviceArray.from_numpy(ctx, v_img))
+    f = ctx.frame()
+    red = oracle.reduce_slots(n, b, oracle.raster_backward(b, fwd, cam, BG, v_img))
+    number = np.isfinite(sc["opac"][:, 0])
+    for k, ptr, shape in (("v_xy", f.v_xy, (n, 2)), ("v_conic", f.v_conic, (n, 3)), ("v_rgb", f.v_rgb, (n, 3)),
+                          ("v_opac", f.v_opacity, (n,))):
+        got, want = ctx.download(ptr, shape, np.float32), red[k].reshape(shape)
+        if k == "v_opac":
+            got, want = got[number], want[number]
+        assert np.isfinite(got).all() and _rel(got, want) < 1e-4, k
+    ctx.close()
