@@ -185,8 +185,9 @@ struct Composite {
 // falls, so when it ends above T_MIN in every pixel of the wave none did, and the colours
 // follow without a test per record. Otherwise (a pixel terminates once) the group is
 // composited step by step: skip (invalid), accept, or terminate (transmittance would drop
-// to T_MIN: last = k - 1, as the CPU).
-template <bool AUX>
+// to T_MIN: last = k - 1, as the CPU). A chunk's pixels that terminated in an earlier one
+// (CHUNK) start at or below T_MIN with every alpha zero, and don't count.
+template <bool AUX, bool CHUNK = false>
 __device__ inline void composite_batch(const float4 *la, const float4 *lb, const float4 *lc, int n8, float fx,
                                        const float (&fy)[FPT], Composite &p) {
 #pragma clang fp contract(fast)
@@ -209,7 +210,7 @@ __device__ inline void composite_batch(const float4 *la, const float4 *lb, const
             }
         }
 #pragma unroll
-        for (int k = 0; k < FPT; k++) low = low || T[k] <= T_MIN;
+        for (int k = 0; k < FPT; k++) low = low || (T[k] <= T_MIN && !(CHUNK && p.done[k]));
         if (__ballot(low) == 0) {
 #pragma unroll
             for (int u = 0; u < G; u++) {
@@ -427,7 +428,7 @@ __device__ inline void forward_chunk(const TileView &v, const TileData &d, const
                 if (__ballot(!p.all_done()) == 0) break;
             }
         } else {
-            composite_batch<false>(la, lb, lc, n8, fx, fy, p);
+            composite_batch<false, true>(la, lb, lc, n8, fx, fy, p);
         }
     }
 #pragma unroll
