@@ -111,8 +111,8 @@ __device__ constexpr float E_MAX = SIGMA_MAX * POW_ONE;
 // position), (r, g, b, view depth), colours stored as composited, max(raw + 0.5, 0).
 // Pixels per record cost three wide reads instead of five narrower ones.
 __device__ inline uint32_t splat_limit(float opacity) {
-    if (opacity < ALPHA_MIN) return 0u;  // nothing is below: never valid
-    if (!(opacity >= ALPHA_MIN)) return __float_as_uint(E_MAX);  // NaN: alpha is min(ALPHA_MAX, NaN) = ALPHA_MAX
+    opacity = fminf(opacity, 2.f);  // a NaN is 2: alpha is min(ALPHA_MAX, NaN) = ALPHA_MAX up to E_MAX
+    if (!(opacity >= ALPHA_MIN)) return 0u;  // nothing is below: never valid
     // the logarithm's own rounding, half a unit of e, decided 18% more pairs wrongly (against
     // 64 bits) than opacity 2^-e >= ALPHA_MIN does: the last bits are taken by that test
     const uint32_t l = max(__float_as_uint(fmaxf(__builtin_amdgcn_logf(opacity * (1.f / ALPHA_MIN)), 0.f)), 2u) - 2u;
