@@ -493,7 +493,11 @@ __device__ inline float mul_or_zero(float a, float b) {
     return r;
 }
 
-constexpr int NPART = 12;  // a record's wave sums in LDS: R0, M, N, four rows each
+constexpr int NPART = 12;  // a record's wave sums: R0, M, N, four rows each
+struct alignas(16) PartSums {  // in LDS; R0 and M are read back as float4
+    float v[NPART];
+};
+static_assert(alignof(PartSums) == 16 && sizeof(PartSums) == 4 * NPART, "whole float4s, side by side");
 struct WaveSums {
     float r0, m, n;
 };
@@ -529,7 +533,7 @@ __device__ inline void backward_tile(const TileView &v, const TileData &d, int g
     __shared__ uint32_t lslot[BATCH];
     __shared__ uint8_t lmask[BATCH];  // bit c: raw colour c + 0.5 >= 0 (its gradient passes)
     __shared__ uint32_t ltouch[NW][(BATCH + 31) / 32];  // per wave, bit j: it had a valid pair with record j
-    __shared__ float part[NW][BATCH][NPART];
+    __shared__ PartSums part[NW][BATCH];
     __shared__ int smax[NW];
     __shared__ int wcount[2][NW];
     __shared__ int lclamp;  // some staged record's opacity reaches ALPHA_MAX: alphas may be clamped
@@ -623,7 +627,7 @@ __device__ inline void backward_tile(const TileView &v, const TileData &d, int g
             kept += total;
         }
         if (NW > 1)  // one wave writes its sums only to the records it reads them back from
-            for (int i = threadIdx.x; i < NW * NPART * BATCH; i += NT) (&part[0][0][0])[i] = 0.f;
+            for (int i = threadIdx.x; i < NW * BATCH * NPART; i += NT) ((float *)part)[i] = 0.f;
         __syncthreads();
         // Per pixel, an invalid pair has alpha 0, which leaves T (times 1 / (1 - 0)) and S as
         // they are and adds zeros (vs by the product that is 0 whenever a factor is). Most
@@ -672,7 +676,7 @@ __device__ inline void backward_tile(const TileView &v, const TileData &d, int g
                     const int c = lane & 15;
                     float sum = c == 0 ? t.r0 : c == 1 ? t.m : t.n;
                     asm volatile("" : "+v"(sum));  // the last row step before the branch, not in it
-                    if (c < 3) part[w][j][4 * c + (lane >> 4)] = sum;
+                    if (c < 3) part[w][j].v[4 * c + (lane >> 4)] = sum;
 #pragma unroll
                     for (int i = 0; i < (BATCH + 31) / 32; i++) touched[i] |= (j >> 5) == i ? 1u << (j & 31) : 0u;
                 }
@@ -691,15 +695,15 @@ __device__ inline void backward_tile(const TileView &v, const TileData &d, int g
             for (int r = 0; r < NW; r++) any |= ltouch[r][j >> 5];
             if (!((any >> (j & 31)) & 1u)) continue;  // every wave's partials are zero
             nwritten++;
-            float4 R0 = *(const float4 *)&part[0][j][0], M = *(const float4 *)&part[0][j][4];
-            float n0 = part[0][j][8], n2 = part[0][j][10];
+            float4 R0 = *(const float4 *)&part[0][j].v[0], M = *(const float4 *)&part[0][j].v[4];
+            float n0 = part[0][j].v[8], n2 = part[0][j].v[10];
 #pragma unroll
             for (int r = 1; r < NW; r++) {
-                const float4 R = *(const float4 *)&part[r][j][0], m = *(const float4 *)&part[r][j][4];
+                const float4 R = *(const float4 *)&part[r][j].v[0], m = *(const float4 *)&part[r][j].v[4];
                 R0.x += R.x; R0.y += R.y; R0.z += R.z; R0.w += R.w;
                 M.x += m.x; M.y += m.y; M.z += m.z; M.w += m.w;
-                n0 += part[r][j][8];
-                n2 += part[r][j][10];
+                n0 += part[r][j].v[8];
+                n2 += part[r][j].v[10];
             }
             // sums of vs: R0.x; dx vs: M.x; dy vs: R0.z; dx^2: n0; dx dy: M.z; dy^2: R0.y; colours R0.w, M.y, M.w
             const float4 Q = lconic[j];  // the unscaled conic (a, b, c)
