@@ -486,7 +486,9 @@ __device__ inline void forward_chunk(const TileView &v, const TileData &d, const
 //   R0, M = (dx q0, q7, dx q2, q8), N = dx^2 R0 (row 0; row 2 carries the depth sum q9).
 // 28 instructions against 38 for a butterfly over the nine values.
 // a * b, and 0 whenever a factor is 0 (also against an infinity or a NaN): a pixel whose
-// upstream gradient is not finite leaves the records it does not see as they are
+// upstream gradient is not finite leaves the positions, conics and opacities of the records
+// it does not see as they are. Their colour and depth sums, 0 times that gradient, become NaN
+// where the pixel's wave adds them up for another pixel.
 __device__ inline float mul_or_zero(float a, float b) {
     float r;
     asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
