@@ -2,9 +2,9 @@
 // render / train / backward pipelines over the gfx950 kernels.
 //
 // A context owns one stream and a grow-only workspace: per-gaussian projection records,
-// per-intersection keys/ids/gradient slots, per-tile ranges and per-pixel buffers. The
+// per-intersection list ids and gradient slots, per-tile ranges and per-pixel buffers. The
 // intersection count is read back once per view (after the per-block count scan) to
-// size the sort; everything else stays on the device.
+// size the lists; everything else stays on the device.
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -32,6 +32,15 @@ int msplat::set_error(int code, const char *fmt, ...) {
 
 namespace {
 
+// The context's device scalars, zero at first
+int make_scalars(msplat_hip_ctx *ctx) {
+    if (ctx->scalars.p) return MSPLAT_OK;
+    CHECKED(ctx->grow(ctx->scalars, 128));
+    zero_u32<<<1, 256, 0, ctx->stream>>>((uint32_t *)ctx->scalars.p, 32);
+    HIPCHECK(hipGetLastError());
+    return MSPLAT_OK;
+}
+
 // projection (per-block intersection and visible counts)
 int do_project(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, const msplat_hip_camera *cam,
                const StepParams *sp = nullptr) {
@@ -51,10 +60,7 @@ int do_project(msplat_hip_ctx *ctx, const msplat_hip_gaussians *g, const msplat_
     CHECKED(ctx->grow(ctx->offsets, 4 * N));
     CHECKED(ctx->grow(ctx->block_sums, 4 * (size_t)(nblocks + 1)));
     CHECKED(ctx->grow(ctx->block_vis, 4 * (size_t)(nblocks + 1)));
-    if (!ctx->scalars.p) {
-        CHECKED(ctx->grow(ctx->scalars, 128));
-        zero_u32<<<1, 256, 0, ctx->stream>>>((uint32_t *)ctx->scalars.p, 32);
-    }
+    CHECKED(make_scalars(ctx));
     CHECKED(ctx->grow(ctx->big, 40 * N + 64));  // list (4) + slot sums (16 + 16 + 4) + alignment
     ctx->n = n;
     ctx->width = cam->width;
@@ -1162,7 +1168,7 @@ int msplat_hip_radix_sort(msplat_hip_ctx *ctx, uint64_t *keys, int32_t *vals, ui
     CHECKED(ctx->grow(ctx->vals1, 4 * (size_t)n));
     CHECKED(ctx->grow(ctx->hist, 4 * radix_hist_words(n)));
     CHECKED(ctx->grow(ctx->digit_total, 4 * 256));
-    CHECKED(ctx->grow(ctx->scalars, 64));
+    CHECKED(make_scalars(ctx));
     uint32_t *dn = ctx->d_total32();
     fill_u32<<<1, 1, 0, ctx->stream>>>(dn, n);
     uint64_t *kin = keys, *kout = (uint64_t *)ctx->keys1.p;

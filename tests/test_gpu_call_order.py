@@ -107,3 +107,27 @@ def test_lists_are_offered_for_a_binned_frame_only():
         assert not f.isect_gid and not f.isect_keys
     finally:
         ctx.close()
+
+
+def test_a_sort_before_the_first_frame():
+    """A radix sort as a context's first call leaves the running counts of its frames zero and
+    all of them allocated (it needs only the element count among those scalars)."""
+    from msplat._abi import Context, DeviceArray, check, lib
+    from msplat.backend import DeviceGaussians, render_numpy
+    sc, cam = _scene()
+    ctx = Context(0)
+    try:
+        keys = DeviceArray.from_numpy(ctx, np.arange(100, 0, -1, dtype=np.uint64))
+        vals = DeviceArray.from_numpy(ctx, np.arange(100, dtype=np.int32))
+        check(lib().msplat_hip_radix_sort(ctx.ptr, C.c_void_p(keys.ptr), C.c_void_p(vals.ptr), 100, 32))
+        np.testing.assert_array_equal(vals.numpy(), np.arange(99, -1, -1, dtype=np.int32))
+        dg = DeviceGaussians(ctx, sc)
+        for frames in range(3):
+            f = ctx.frame()
+            assert ctx.download(f.isects_running, (1,), np.uint64)[0] == frames * f.num_isects
+            assert ctx.download(f.visible_running, (1,), np.uint64)[0] == frames * f.num_visible
+            assert ctx.download(f.slots_written, (1,), np.uint64)[0] == 0
+            render_numpy(ctx, dg, cam, BG)
+        assert ctx.frame().num_isects > 0
+    finally:
+        ctx.close()
