@@ -455,8 +455,7 @@ std::vector<uint64_t> shape_key(msplat_hip_ctx *ctx, const StepRecord &r) {
                                bits(r.inv_max), bits(r.adam.beta1), bits(r.adam.beta2), bits(r.adam.eps),
                                (uint64_t)ctx->flags, (uint64_t)ctx->tuning.chunks, (uint64_t)ctx->tuning.bwd_ppt,
                                (uint64_t)ctx->tuning.fwd_batch, (uint64_t)ctx->tuning.bwd_batch,
-                               (uint64_t)ctx->tuning.cull, (uint64_t)ctx->tuning.pack_keys,
-                               (uint64_t)(uintptr_t)r.radii_out};
+                               (uint64_t)ctx->tuning.cull, (uint64_t)(uintptr_t)r.radii_out};
     const void *ptrs[] = {r.g.means, r.g.scales, r.g.quats, r.g.features_dc, r.g.features_rest, r.g.opacities,
                           r.stats.vis_counts, r.stats.xys_grad_norm, r.stats.max_2d_size};
     for (const void *p : ptrs) k.push_back((uint64_t)(uintptr_t)p);

@@ -457,12 +457,11 @@ __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kou
     const uint32_t wstart = start + (uint32_t)w * (64 * R);
     K key[R];
     int32_t val[R];
-    const bool has_vals = vin != nullptr;  // null: the keys carry their payload
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const uint32_t e = wstart + r * 64 + lane;
         key[r] = e < n ? kin[e] : K(0);
-        val[r] = has_vals && e < n ? vin[e] : 0;
+        val[r] = e < n ? vin[e] : 0;
     }
     wave_sync();
     // per element: digit (bits 24..31) and rank among the wave's elements of that digit
@@ -502,7 +501,7 @@ __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kou
         if (wstart + r * 64 + lane < n) {
             const uint32_t p = wcnt[w][dr[r] >> 24] + (dr[r] & 0xFFFFFF);
             sk[p] = key[r];
-            if (has_vals) sv[p] = val[r];
+            sv[p] = val[r];
         }
     }
     __syncthreads();
@@ -511,18 +510,16 @@ __device__ inline void rs_scatter_block(const K *kin, const int32_t *vin, K *kou
         const K k = sk[p];
         const uint32_t d = (uint32_t)(k >> shift) & mask;
         const uint32_t o = gbase[d] + (p - lstart[d]);
+        const int32_t v = sv[p];
+        vout[o] = v;
         if (entries.lrect) {
-            const int32_t v = sv[p];
             const uint2 q = entries.rect[v];
-            vout[o] = v;
             entries.lrect[o] = entries.direct ? make_uint2((uint32_t)v, pack_local(q, 0, 0)) : q;
-            continue;
+        } else {
+            kout[o] = k;
         }
-        kout[o] = k;
-        if (has_vals) vout[o] = sv[p];
     }
 }
-
 
 template <typename K, int ITEMS>
 __global__ __launch_bounds__(256) void rs_scatter_kernel(const K *kin, const int32_t *vin, K *kout, int32_t *vout,

@@ -56,23 +56,11 @@ __device__ inline void tile_rect(float cx, float cy, float rx, float ry, int tx,
     y1 = min(max(0, (int)(ccy + rry + 1.f)), ty);
 }
 
-// ── wave64 sum over DPP ────────────────────────────────────────────────────
-// Lanes of a 16-lane row are combined by quad permutes and the row (half-)mirrors,
-// the four rows by row broadcasts; the total ends in lane 63 and is returned as a
-// wave-uniform value.
-template <int CTRL, int ROW_MASK = 0xf>
+// ── wave64 sums over DPP: quad permutes and the row (half-)mirrors combine the lanes of a
+// 16-lane row ─────────────────────────────────────────────────────────────────
+template <int CTRL>
 __device__ inline float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
-}
-
-__device__ inline float wave_sum(float v) {
-    v += dpp_f<0xb1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_f<0x4e>(v);   // quad_perm [2,3,0,1]
-    v += dpp_f<0x141>(v);  // row_half_mirror
-    v += dpp_f<0x140>(v);  // row_mirror
-    v += dpp_f<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    v += dpp_f<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
 // Sum over the 16 lanes of each DPP row; every lane of the row ends with the row total.
@@ -81,13 +69,6 @@ __device__ inline float row_sum16(float v) {
     v += dpp_f<0x4e>(v);   // quad_perm [2,3,0,1]
     v += dpp_f<0x141>(v);  // row_half_mirror
     v += dpp_f<0x140>(v);  // row_mirror
-    return v;
-}
-
-// Completes a row_sum16: lane 63 ends with the total of the four rows' sums.
-__device__ inline float rows_to_lane63(float v) {
-    v += dpp_f<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    v += dpp_f<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
     return v;
 }
 
@@ -158,8 +139,6 @@ __device__ inline float wave_sums10(const SumLanes &L, float q0, float q1, float
     e += dpp_f<0x140>(e);
     return sum_rows(L.q == 8 ? e : u);
 }
-
-__device__ inline uint64_t ballot(bool p) { return __ballot(p); }
 
 // A tile rectangle (x0 | x1 << 16, y0 | y1 << 16) within the supertile of 8x8 tiles at
 // (ox, oy): four 4-bit numbers x0 | x1 << 4 | y0 << 8 | y1 << 12

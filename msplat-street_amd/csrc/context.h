@@ -40,13 +40,6 @@ inline int check_gaussians(const msplat_hip_gaussians *g) {
     return MSPLAT_OK;
 }
 
-inline int tile_bits(int ntiles) {
-    int b = 0;
-    while ((1 << b) < ntiles) b++;
-    return b;
-}
-
-
 }  // namespace msplat
 
 #define HIPCHECK(expr)                                                                                           \
