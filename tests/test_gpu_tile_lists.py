@@ -64,6 +64,44 @@ def test_lists_hold_each_tiles_gaussians_in_depth_order(W, H, n, scale):
     ctx.close()
 
 
+def test_lists_and_keys_at_street_scale():
+    """475,115 gaussians at 1264x832 (4,108 tiles, two level-1 nodes, millions of
+    intersections): the lists, their ranges, and the 64-bit (tile << 32 | depth bits) keys made
+    of them, against the same restatement with the rectangles expanded whole."""
+    from msplat._abi import FRAME_KEYS64, Context
+    from msplat.backend import DeviceGaussians, render
+    from msplat.scenes import street_cameras, street_points
+    n, W, H = 475_115, 1264, 832
+    ctx = Context(0)
+    ctx.set_flags(FRAME_KEYS64)
+    dg = DeviceGaussians.from_points(ctx, *street_points(0, n), degree=0)
+    cam = street_cameras(4, W, H, 900.0, 900.0)[1]
+    render(ctx, dg, cam, BG)
+    f = ctx.frame()
+    M, tx, ty = int(f.num_isects), cam["tiles_x"], cam["tiles_y"]
+    F, t = np.float32, np.array([tx, ty])
+    ids = np.nonzero(ctx.download(f.radii, (n,), np.int32) > 0)[0]
+    dep = ctx.download(f.depths, (n,), np.float32).view(np.uint32)
+    c = ctx.download(f.splat_a, (n, 4), np.float32)[ids, :2] / F(16)
+    r = ctx.download(f.aabb, (n, 2), np.float32)[ids] / F(16)
+    lo, hi = np.clip((c - r).astype(np.int64), 0, t), np.clip((c + r + F(1)).astype(np.int64), 0, t)
+    order = np.lexsort((ids, dep[ids]))
+    ids, lo, size = ids[order], lo[order], np.maximum(hi - lo, 0)[order]
+    count = size[:, 0] * size[:, 1]
+    at = np.repeat(np.arange(ids.size), count)
+    k = np.arange(at.size) - np.repeat(np.cumsum(count) - count, count)
+    tile = (lo[at, 1] + k // size[at, 0]) * tx + lo[at, 0] + k % size[at, 0]
+    by_tile = np.argsort(tile, kind="stable")
+    gids, tile = ids[at[by_tile]], tile[by_tile]
+    assert M == gids.size > 1_000_000
+    np.testing.assert_array_equal(ctx.download(f.tile_start, (tx * ty + 1,), np.int32),
+                                  np.searchsorted(tile, np.arange(tx * ty + 1)))
+    np.testing.assert_array_equal(ctx.download(f.isect_gid, (M,), np.int32), gids)
+    np.testing.assert_array_equal(ctx.download(f.isect_keys, (M,), np.uint64),
+                                  (tile.astype(np.uint64) << np.uint64(32)) | dep[gids].astype(np.uint64))
+    ctx.close()
+
+
 @pytest.mark.parametrize("graph", [False, True])
 def test_batched_lists_give_the_one_view_images(graph):
     """Views of one to nine level-1 nodes in one batch (and one behind the camera): their
