@@ -342,8 +342,10 @@ __global__ __launch_bounds__(256) void compact_kernel(CompactArgs a) {
 // intersections (in no particular order): each workgroup counts those of its part of the
 // records, takes its place in the list with one atomic, and writes them. One atomic per
 // 256 records, as the list was first built, serialised on its counter (about 12 ns each:
-// 21 us at 475k records, 360 us for a batch of 8 views of 1M). 256 workgroups take 9.9 us
-// at 475k and 117 us for the batch, 1024 take 16.7 and 70.
+// 21 us at 475k records, 360 us for a batch of 8 views of 1M). Few workgroups pay less for
+// the atomics, many clear the flags faster. By itself, with 17 slots a record and one record
+// in eight listed, 256 workgroups / 1024: 10.7 / 18.0 us at 475k records, 17.1 / 21.0 at
+// 1.5M, 23.8 / 22.8 at 2M (the line), 31.2 / 25.8 at 3M, 86 / 46 at 8M.
 constexpr size_t SLOT_PREPARE_GRID = 1024;
 constexpr uint32_t SLOT_PREPARE_MANY = 2u << 20;
 __global__ __launch_bounds__(256) void slot_prepare_kernel(SlotPrepareArgs a) {
