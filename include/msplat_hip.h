@@ -188,7 +188,8 @@ int msplat_hip_render_backward(msplat_hip_ctx *ctx, const msplat_hip_gaussians *
  * and tools. Per gaussian: xys (N,2) as float4 records (x, y, conic.x, conic.y) and
  * (conic.z, sigmoid(opacity), r, g) plus blue (N), depths, radii, aabb (N,2), tile
  * counts, prefix offsets (in id order). Per intersection (sorted): keys (tile<<32 | depth
- * bits, filled by frame_view when MSPLAT_FRAME_KEYS64 is set, else NULL), gaussian ids.
+ * bits, filled by frame_view when MSPLAT_FRAME_KEYS64 is set, else NULL), gaussian ids;
+ * both are NULL while the frame is not binned.
  * tile_start (T+1): tile t owns sorted intersections [tile_start[t], tile_start[t+1]).
  * Per pixel: image, final_T, final_idx (index into
  * the sorted intersections), dL/d(image). Per gaussian reduced gradients (N,2)/(N,3)/
@@ -382,8 +383,8 @@ int msplat_hip_pack_rgba8(msplat_hip_ctx *ctx, const float *img, uint32_t n, uin
 /* ── batched views (no reference counterpart: the reference renders and trains one view
  * per call, msplat_render / msplat_train_step, bindings.h:81-118) ──────────────────
  * Several views of one scene, of mixed resolution, in one pass: one projection of every
- * gaussian into every view, one key sort over all views' tiles, a persistent rasterizer
- * that pulls (view, tile) items from a device work queue, one loss pass and one
+ * gaussian into every view, one depth sort and one expansion into every view's tile
+ * lists, a persistent rasterizer that pulls (view, tile) items from a device work queue, one loss pass and one
  * backward that sums the views' gradients. Per view the results equal those of the
  * one-view entry points (images, final T and contributor indices bit for bit;
  * gradients within float rounding of the sum of one-view gradients).

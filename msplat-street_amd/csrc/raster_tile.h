@@ -2,8 +2,8 @@
 // functions shared by the one-view kernels (one workgroup per tile) and the persistent
 // batched kernels (workgroups pull (view, tile) items from a queue).
 //
-// Both are bound by VALU issue (the forward fills it, the backward 85%: its one wave per tile
-// leaves it to the slowest tiles), so what counts is instructions per pixel and record and
+// Both are bound by VALU issue (the forward fills it, the backward uses 75% of it: its one wave
+// per tile leaves the rest to the slowest tiles), so what counts is instructions per pixel and record and
 // the records that are visited at all: 18 instructions in the forward (28 before), 32 in the
 // backward (45). On the 475k street scene at 1264x832 the forward kernel went 211 -> 155 us
 // and the backward 449 -> 362 us, at 3M gaussians and 3840x2160 the forward 381 -> 250 us;
@@ -181,12 +181,16 @@ struct Composite {
 
 // Composites the staged records [0, n8) (n8 a multiple of 8) into the lane's pixels (fx,
 // fy[k]). Groups of G: the alphas first (independent of each other), then the
-// transmittance through the group as if no pixel terminated in it. Transmittance only
-// falls, so when it ends above T_MIN in every pixel of the wave none did, and the colours
-// follow without a test per record. Otherwise (a pixel terminates once) the group is
-// composited step by step: skip (invalid), accept, or terminate (transmittance would drop
-// to T_MIN: last = k - 1, as the CPU). A chunk's pixels that terminated in an earlier one
-// (CHUNK) start at or below T_MIN with every alpha zero, and don't count.
+// transmittance through the group as if no pixel terminated in it, T - alpha T in one
+// rounding. (By the rounded factor 1 - alpha, which the backward divides by again, it takes
+// one instruction more, 1% of a train step, and is no closer to 64 bits: over six scenes
+// each of four cases the median record's gradient error moves by -1 to +2%, images' by +1%.)
+// Transmittance only falls, so when it ends above T_MIN in every pixel of the wave none
+// did, and the colours follow without a test per record. Otherwise (a pixel terminates
+// once) the group is composited step by step: skip (invalid), accept, or terminate
+// (transmittance would drop to T_MIN: last = k - 1, as the CPU). A chunk's pixels that
+// terminated in an earlier one (CHUNK) start at or below T_MIN with every alpha zero, and
+// don't count.
 template <bool AUX, bool CHUNK = false>
 __device__ inline void composite_batch(const float4 *la, const float4 *lb, const float4 *lc, int n8, float fx,
                                        const float (&fy)[FPT], Composite &p) {

@@ -37,7 +37,7 @@ from .backend import BatchViews, DeviceGaussians, render_batch
 
 REC_BYTES = 116    # per record (view x gaussian) of a batched frame
 PIX_BYTES = 40     # per pixel: image, final T and index, gradient image, loss, RGBA8
-ISECT_BYTES = 52   # per intersection: keys, ids (double-buffered), gradient slots
+ISECT_BYTES = 52   # per intersection: list entries (12), gradient slots (37), their share of headroom
 PARAM_BYTES = 236  # per resident SH3 gaussian (59 floats)
 MIN_VIEW = (640, 360)  # the smallest view every slot must keep room for
 
