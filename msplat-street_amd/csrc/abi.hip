@@ -415,7 +415,7 @@ int eager_step_tail(msplat_hip_ctx *ctx, const StepRecord &r) {
     return MSPLAT_OK;
 }
 
-// One train step, launch by launch (the counts are read back to size the key buffers)
+// One train step, launch by launch (the counts are read back to size the list buffers)
 int eager_step(msplat_hip_ctx *ctx, const StepRecord &r, float *loss_out) {
     CHECKED(do_project(ctx, &r.g, &r.cam));
     CHECKED(do_bin(ctx));

@@ -2,9 +2,9 @@
 // functions shared by the one-view kernels (one workgroup per tile) and the persistent
 // batched kernels (workgroups pull (view, tile) items from a queue).
 //
-// Both are bound by VALU issue (the forward fills it, the backward uses 75% of it: its one wave
-// per tile leaves the rest to the slowest tiles), so what counts is instructions per pixel and record and
-// the records that are visited at all: 18 instructions in the forward (28 before), 32 in the
+// Both are bound by VALU issue (the forward fills it, the backward uses 79% of it: its one
+// wave per tile leaves the rest to the slowest tiles), so what counts is instructions per
+// pixel and record and the records that are visited at all: 18 instructions in the forward (28 before), 32 in the
 // backward (45). On the 475k street scene at 1264x832 the forward kernel went 211 -> 155 us
 // and the backward 449 -> 362 us, at 3M gaussians and 3840x2160 the forward 381 -> 250 us;
 // the exact ellipse test in place of the bounding box gives about 15% and 8% of it.

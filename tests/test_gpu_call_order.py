@@ -1,6 +1,6 @@
 """Stage entry points called out of order are refused on the host with MSPLAT_ERR_ARG,
 before any kernel launch: a raster or loss stage with no binned frame, a backward with no
-render, and any of them after msplat_hip_radix_sort reused the frame's key buffers. Each
+render, and any of them after msplat_hip_radix_sort ended the frame. Each
 refusal leaves the context usable: a full render afterwards still matches a fresh one.
 """
 import ctypes as C
@@ -50,7 +50,7 @@ def test_out_of_order_stages_are_refused():
         # binned, not rasterized: the loss and the backward still need an image
         check(L.msplat_hip_stage_bin(ctx.ptr, C.byref(c)))
         assert L.msplat_hip_stage_loss(ctx.ptr, C.byref(c), C.c_void_p(gt.ptr), 0.2, 1e-3, C.byref(loss)) == ERR_ARG
-        # a rendered frame, then a radix sort that reuses its key buffers
+        # a rendered frame, then a radix sort, which ends it
         ref = render_numpy(ctx, dg, cam, BG)
         keys = DeviceArray.from_numpy(ctx, np.arange(100, 0, -1, dtype=np.uint64))
         vals = DeviceArray.from_numpy(ctx, np.arange(100, dtype=np.int32))

@@ -92,10 +92,9 @@ def test_binning_bit_exact_on_oracle_inputs(ctx, oracle, ties):
 
 
 def test_binning_bit_exact_with_huge_splats(ctx, oracle):
-    """Key emission across its 2048-key workgroup slices: at 1920x1080 (8160 tiles) a few
-    splats cover most of the image, so their keys span several slices and slices start
-    inside them, among thousands of small splats whose records start anywhere in a
-    thread's eight outputs."""
+    """Records from under a tile to most of 1920x1080's 8160 tiles: a few splats of thousands
+    of intersections each, so that they are in most supertiles' lists whole, among thousands
+    of small ones."""
     from msplat.camera import look_at, make_camera
     from msplat.scenes import random_scene
     sc = random_scene(9, 4000, degree=1, log_scale=(-3.5, 0.5))
