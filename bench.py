@@ -1214,7 +1214,7 @@ def main():
         "mpix_per_s": round(P * iters / 1e6, 1),
         "sh_degree_in_use": dtu_timed,
     }
-    # HBM rate of every stage over the stage window, by the per-unit formulas
+    # HBM rate of every stage over the stage window
     ns = max(args.stage_steps, 1)
     sM, sV, sN, sB = sw["M"] / ns, sw["V"] / ns, sw["N"] / ns, sw["B"] / ns
     stage_rows = {}
@@ -1223,12 +1223,11 @@ def main():
             continue
         per = ms / calls
         b8, bb = alg_bytes_8d(k, sM, sV, sN, P, T, sB), alg_bytes_build(k, sM, sV, sN, P, T, sB)
-        # the share of the peak is by this build's own bytes: by the other count, a stage that
-        # moves fewer could exceed it
-        stage_rows[k] = {"ms": round(per, 4), "bytes": int(b8), "gbs": round(b8 / (per * 1e-3) / 1e9, 1),
+        # by this build's own bytes: by the plan's, a stage that moves fewer could exceed the peak
+        stage_rows[k] = {"ms": round(per, 4), "bytes": int(bb), "gbs": round(bb / (per * 1e-3) / 1e9, 1),
                          "frac": round(bb / (per * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
         if bb != b8:
-            stage_rows[k].update(build_bytes=int(bb), build_gbs=round(bb / (per * 1e-3) / 1e9, 1))
+            stage_rows[k]["plan_bytes"] = int(b8)
     roofline["stages"] = stage_rows
     roofline["stages_window"] = {"steps": args.stage_steps, "intersections": int(sM), "visible": int(sV),
                                  "gaussians": int(sN), "sh_bases": round(sB, 2)}
